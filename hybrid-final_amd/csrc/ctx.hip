@@ -407,10 +407,6 @@ struct Case : CaseBase {
             HIPCHK(hipMemsetAsync(x64, 0, std::max(1, N) * sizeof(double), st));
             HIPCHK(hipMemsetAsync(b64, 0, std::max(1, N) * sizeof(double), st));
             op.N = N; op.col = pcol; op.valf = pvalf; op.vald = pvald; op.mdiagf = pmdf; op.mdiagd = pmdd;
-            int werr = 0;
-            const char *nb_env = getenv("PIC_PCG_BLOCKS");
-            pw = pcg_work_create(N, &werr, nb_env ? atoi(nb_env) : 0, st);
-            if (!pw) return fail(-40, "field solver workspace allocation failed");
             HIPCHK(dalloc(&d_res, 1));
             HIPCHK(hipMemsetAsync(d_res, 0, sizeof(PcgResult), st));
             if ((precision == PIC_FP32_REFINED && field_solver == 0) || field_solver == 2) {
@@ -451,12 +447,17 @@ struct Case : CaseBase {
                     solver_kind = 1;
                 }
             }
-        }
-        // the persistent solver's launch shape, tuned on this operator when
-        // the PCG is the field solver (PIC_PCG_BLOCKS fixes the grid instead)
-        if (!spectral && !getenv("PIC_PCG_BLOCKS") && S.A_size > 0) {
-            if (int e2 = pcg_autotune(pw, op, precision == PIC_FP32_REFINED, st, nullptr))
-                return fail(e2, "field solver autotuning failed");
+            // the PCG's work space and launch shape (PIC_PCG_BLOCKS fixes the
+            // grid), where the PCG is the field solver
+            if (!spectral) {
+                int werr = 0;
+                const char *nb_env = getenv("PIC_PCG_BLOCKS");
+                pw = pcg_work_create(N, col.data(), vd.data(), &werr, nb_env ? atoi(nb_env) : 0, st);
+                if (!pw) return fail(-40, "field solver workspace allocation failed");
+                if (!nb_env && N > 0)
+                    if (int e2 = pcg_autotune(pw, op, precision == PIC_FP32_REFINED, st, nullptr))
+                        return fail(e2, "field solver autotuning failed");
+            }
         }
         // particles
         int capmax = 0;
@@ -615,15 +616,15 @@ struct Case : CaseBase {
     }
     // the solve itself: FP64 solution in x64 (warm start) from the rhs brhs
     int solve_x64() {
-        const int N = S.A_size;
         const double tol = S.deck.pcg_tol > 0 ? S.deck.pcg_tol : 1e-10;
         if (spectral) {
             // the first residual converts the rhs into b64
             spectral_solve_refined<R>(op, spec, brhs, b64, x64, tol, spec_cycles, spec_state, spec_part, d_res, st);
         } else {
-            launch_rhs_to_fp64<R>(N, brhs, b64, st);
-            if (precision == PIC_FP64_PLAIN) HIPCHK(pcg_solve_plain_fp64(op, b64, x64, tol, pcg_maxit, pw, d_res, st));
-            else HIPCHK(pcg_solve_refined(op, b64, x64, tol, inner_tol, pcg_maxit, pw, d_res, st));
+            if constexpr (std::is_same<R, double>::value)
+                HIPCHK(pcg_solve_plain_fp64(op, brhs, x64, tol, pcg_maxit, pw, d_res, st));
+            else
+                HIPCHK(pcg_solve_refined(op, brhs, b64, x64, tol, inner_tol, pcg_maxit, pw, d_res, st));
         }
         HIPCHK(hipGetLastError());
         return 0;

@@ -1,5 +1,7 @@
-// Field solve: Jacobi-preconditioned conjugate gradients as one persistent
-// kernel per solve (the reference's PCG_float,
+// Field solve: Jacobi-preconditioned conjugate gradients.  Operators whose
+// vectors fit the registers of at most half the CUs are solved by the kernels
+// of pcg_resident.hip; the ones here keep the vectors in memory and take any
+// size, as one persistent kernel per solve (the reference's PCG_float,
 // src/cuda_Field.cu:942-1072, uses the same single-launch structure).
 //
 //  * plain FP64 path: vectors, operator and dot products in FP64;
@@ -20,6 +22,7 @@
 #include <mutex>
 #include <vector>
 
+#include "pcg_resident.h"
 #include "pic_kernels.h"
 
 namespace pic {
@@ -44,6 +47,7 @@ struct PcgWork {
     double *partials = nullptr;   // 2 sets x PCG_MAX_BLOCK x PCG_NRED
     GridSync *gs = nullptr;
     unsigned long long spin_limit = 0;   // barrier wait limit, in ticks of the 100 MHz constant clock
+    PcgResident *resident = nullptr;     // the register-resident solver, where the operator is in its range
 };
 
 namespace {
@@ -361,7 +365,7 @@ static int pcg_resident_per_cu(int bs) {
     return a < b ? a : b;
 }
 
-PcgWork *pcg_work_create(int N, int *err, int want_blocks, hipStream_t stream) {
+PcgWork *pcg_work_create(int N, const int *col, const double *val, int *err, int want_blocks, hipStream_t stream) {
     PcgWork *w = new PcgWork();
     w->N = N;
     int dev = 0, ncu = 0;
@@ -397,7 +401,19 @@ PcgWork *pcg_work_create(int N, int *err, int want_blocks, hipStream_t stream) {
     // became resident together (PIC_PCG_SPIN_US overrides, for tests of the
     // abandon path)
     w->spin_limit = 200000000ull;
-    if (const char *sl = getenv("PIC_PCG_SPIN_US")) w->spin_limit = 100ull * strtoull(sl, nullptr, 10);
+    const char *sl = getenv("PIC_PCG_SPIN_US");
+    if (sl) w->spin_limit = 100ull * strtoull(sl, nullptr, 10);
+    // a wait limit is only seen by a solve that waits: it asks for several blocks
+    w->resident = pcg_resident_create(N, col, val, ncu, want_blocks, sl != nullptr, stream, err);
+    if (*err) {
+        delete w;
+        return nullptr;
+    }
+    if (w->resident) {
+        w->nblk = w->resident->nblk;
+        w->bs = w->resident->bs;
+        return w;
+    }
     size_t n = (size_t)N;
     hipError_t e = hipSuccess;
     e = (hipError_t)(e | hipMalloc(&w->r, n * sizeof(double)));
@@ -427,6 +443,7 @@ PcgWork *pcg_work_create(int N, int *err, int want_blocks, hipStream_t stream) {
 
 void pcg_work_destroy(PcgWork *w) {
     if (!w) return;
+    pcg_resident_destroy(w->resident);
     void *bufs[] = {w->r, w->z, w->p, w->q, w->rf, w->zf, w->pf, w->qf, w->df, w->partials, w->gs};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
@@ -436,6 +453,7 @@ void pcg_work_destroy(PcgWork *w) {
 int pcg_grid_blocks(PcgWork *w) { return w ? w->nblk : 0; }
 
 hipError_t pcg_work_reset(PcgWork *w, hipStream_t s) {
+    if (w->resident) return pcg_resident_reset(w->resident, s);
     hipLaunchKernelGGL(k_pcg_reset, dim3(1), dim3(64), 0, s, w->gs);
     return hipGetLastError();
 }
@@ -455,6 +473,7 @@ static void launch_refined(const PcgOperator &A, const double *b, double *x, dou
 
 hipError_t pcg_solve_plain_fp64(const PcgOperator &A, const double *b, double *x, double tol, int maxit, PcgWork *w,
                                 PcgResult *res, hipStream_t s) {
+    if (w->resident) return pcg_resident_plain(w->resident, A, b, x, tol, maxit, w->spin_limit, res, s);
     switch (w->bs) {
     case 128: launch_plain<128>(A, b, x, tol, maxit, w, res, s); break;
     case 512: launch_plain<512>(A, b, x, tol, maxit, w, res, s); break;
@@ -463,14 +482,22 @@ hipError_t pcg_solve_plain_fp64(const PcgOperator &A, const double *b, double *x
     return hipGetLastError();
 }
 
-hipError_t pcg_solve_refined(const PcgOperator &A, const double *b, double *x, double tol, double inner_tol,
-                             int maxit, PcgWork *w, PcgResult *res, hipStream_t s) {
+static hipError_t solve_refined64(const PcgOperator &A, const double *b, double *x, double tol, double inner_tol,
+                                  int maxit, PcgWork *w, PcgResult *res, hipStream_t s) {
     switch (w->bs) {
     case 128: launch_refined<128>(A, b, x, tol, inner_tol, maxit, w, res, s); break;
     case 512: launch_refined<512>(A, b, x, tol, inner_tol, maxit, w, res, s); break;
     default: launch_refined<256>(A, b, x, tol, inner_tol, maxit, w, res, s); break;
     }
     return hipGetLastError();
+}
+
+hipError_t pcg_solve_refined(const PcgOperator &A, const float *b, double *b64, double *x, double tol,
+                             double inner_tol, int maxit, PcgWork *w, PcgResult *res, hipStream_t s) {
+    if (w->resident)
+        return pcg_resident_refined(w->resident, A, b, x, tol, inner_tol, maxit, w->spin_limit, res, s);
+    launch_rhs_to_fp64<float>(A.N, b, b64, s);
+    return solve_refined64(A, b64, x, tol, inner_tol, maxit, w, res, s);
 }
 
 // Autotuner of the persistent solver's launch shape: threads per block
@@ -487,6 +514,10 @@ static std::mutex g_tune_mu;
 static std::map<TuneKey, std::pair<int, int>> g_tune;
 
 int pcg_autotune(PcgWork *w, const PcgOperator &A, int refined, hipStream_t st, double *best_us_per_iter) {
+    if (w->resident) {   // its shape follows from the unknowns
+        if (best_us_per_iter) *best_us_per_iter = 0.0;
+        return 0;
+    }
     const TuneKey key{w->N, refined ? 1 : 0};
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -535,7 +566,7 @@ int pcg_autotune(PcgWork *w, const PcgOperator &A, int refined, hipStream_t st, 
             for (int rep = 0; rep < 2 && rc == 0; ++rep) {
                 if (hipMemsetAsync(x, 0, (size_t)N * sizeof(double), st) != hipSuccess ||
                     hipEventRecord(e0, st) != hipSuccess) { rc = -40; break; }
-                const hipError_t le = refined ? pcg_solve_refined(A, b, x, 0.0, 0.0, iters, w, res, st)
+                const hipError_t le = refined ? solve_refined64(A, b, x, 0.0, 0.0, iters, w, res, st)
                                               : pcg_solve_plain_fp64(A, b, x, 0.0, iters, w, res, st);
                 if (le != hipSuccess || hipEventRecord(e1, st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                     hipEventElapsedTime(&ms, e0, e1) != hipSuccess) { rc = -40; break; }

@@ -195,7 +195,8 @@ struct PcgOperator {
 };
 
 struct PcgWork;   // device scratch owned by the context
-PcgWork *pcg_work_create(int N, int *err, int want_blocks, hipStream_t stream);
+// col, val: the operator's 5N columns and values (host)
+PcgWork *pcg_work_create(int N, const int *col, const double *val, int *err, int want_blocks, hipStream_t stream);
 void pcg_work_destroy(PcgWork *);
 int pcg_grid_blocks(PcgWork *);
 // per-step diagnostics (diag.hip)
@@ -240,12 +241,12 @@ hipError_t pcg_work_reset(PcgWork *, hipStream_t);
 int pcg_autotune(PcgWork *, const PcgOperator &A, int refined, hipStream_t st, double *best_us_per_iter);
 int pcg_launch_shape(const PcgWork *, int *blocks, int *threads);
 
-// x (FP64, warm start, in/out), b (FP64).  Writes the result to *res (device
-// memory) so the solve can run inside a captured graph.
+// x (FP64, warm start, in/out).  Writes the result to *res (device memory).
+// The refined solve takes the FP32 right-hand side; b64 is its work array.
 hipError_t pcg_solve_plain_fp64(const PcgOperator &A, const double *b, double *x, double tol, int maxit, PcgWork *w,
                                 PcgResult *res, hipStream_t s);
-hipError_t pcg_solve_refined(const PcgOperator &A, const double *b, double *x, double tol, double inner_tol,
-                             int maxit, PcgWork *w, PcgResult *res, hipStream_t s);
+hipError_t pcg_solve_refined(const PcgOperator &A, const float *b, double *b64, double *x, double tol,
+                             double inner_tol, int maxit, PcgWork *w, PcgResult *res, hipStream_t s);
 
 // ---- separable fast solve (spectral.hip), FP64 throughout
 struct SpecDev {
