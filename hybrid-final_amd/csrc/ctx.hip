@@ -130,7 +130,8 @@ struct Case : CaseBase {
     SpecState *spec_state = nullptr;
     double *spec_part = nullptr;
     std::vector<double *> spec_bufs;
-    int spec_cycles = 1;
+    int spec_cycles = 1, spec_kind = 1;
+    SpecFinal spec_fin{};   // the last solve's convergence test, left to the fused step's kernels
     // particles: two buffers per species
     PView<R> cur[MAXSP]{}, nxt[MAXSP]{};
     uint8_t *tag[MAXSP] = {nullptr};
@@ -414,6 +415,7 @@ struct Case : CaseBase {
                 std::string why;
                 if (build_spectral<R>(S, sp, why)) {
                     const int nx = sp.nx, ny = sp.ny;
+                    spec.nx = nx; spec.ny = ny;
                     std::vector<double> VyiT((size_t)ny * ny), VyT((size_t)ny * ny), dinv((size_t)nx * ny);
                     for (int a = 0; a < ny; ++a)
                         for (int b2 = 0; b2 < ny; ++b2) {
@@ -422,27 +424,30 @@ struct Case : CaseBase {
                         }
                     for (int a = 0; a < nx; ++a)
                         for (int b2 = 0; b2 < ny; ++b2) {
-                            double den = sp.cx * sp.lx[a] + sp.cy * sp.ly[b2];
+                            const double den = sp.cx * sp.lx[a] + sp.cy * sp.ly[b2] + sp.shift;
                             dinv[(size_t)a * ny + b2] = den > 1e-300 ? 1.0 / den : 0.0;
                         }
                     double *p;
                     const std::vector<double> *srcs[5] = {&sp.Vxi, &VyiT, &sp.Vx, &VyT, &dinv};
-                    const double *dst[5];
+                    const double **dst[5] = {&spec.Vxi, &spec.VyiT, &spec.Vx, &spec.VyT, &spec.dinv};
                     for (int q = 0; q < 5; ++q) {
                         HIPCHK(upload(&p, *srcs[q], st));
                         spec_bufs.push_back(p);
-                        dst[q] = p;
+                        *dst[q] = p;
                     }
-                    spec.nx = nx; spec.ny = ny;
-                    spec.Vxi = dst[0]; spec.VyiT = dst[1]; spec.Vx = dst[2]; spec.VyT = dst[3]; spec.dinv = dst[4];
-                    HIPCHK(dalloc(&p, (size_t)nx * ny)); spec_bufs.push_back(p); spec.T1 = p;
-                    HIPCHK(dalloc(&p, (size_t)nx * ny)); spec_bufs.push_back(p); spec.T2 = p;
-                    HIPCHK(dalloc(&p, (size_t)nx * ny)); spec_bufs.push_back(p); spec.r = p;
+                    for (double **w : {&spec.T1, &spec.T2, &spec.r}) {
+                        HIPCHK(dalloc(&p, (size_t)nx * ny));
+                        spec_bufs.push_back(p);
+                        *w = p;
+                    }
                     HIPCHK(dalloc(&spec_state, 1));
-                    HIPCHK(dalloc(&spec_part, 2 * ((N + 255) / 256) + 2));
+                    HIPCHK(hipMemsetAsync(spec_state, 0, sizeof(SpecState), st));
+                    HIPCHK(dalloc(&spec_part, 2 * (size_t)std::max((N + 255) / 256, field_partials(G))));
                     // an exact separable model converges in one FP64 cycle; otherwise
                     // the model error (~1e-7 relative) needs a few refinement cycles
                     spec_cycles = sp.exact ? 1 : 4;
+                    // a batch takes cases of one kind: exact without a shift, or not
+                    spec_kind = sp.exact && !sp.shifted ? 1 : 4;
                     spectral = true;
                     solver_kind = 1;
                 }
@@ -614,12 +619,14 @@ struct Case : CaseBase {
         clk_dirty = false;
         return 0;
     }
-    // the solve itself: FP64 solution in x64 (warm start) from the rhs brhs
+    // the solve itself: FP64 solution in x64 (warm start) from the rhs brhs;
+    // the separable solve leaves its last convergence test to the caller
     int solve_x64() {
         const double tol = S.deck.pcg_tol > 0 ? S.deck.pcg_tol : 1e-10;
+        spec_fin = SpecFinal{};
         if (spectral) {
-            // the first residual converts the rhs into b64
-            spectral_solve_refined<R>(op, spec, brhs, b64, x64, tol, spec_cycles, spec_state, spec_part, d_res, st);
+            spec_fin = spectral_solve<R>(op, spec, (const R *)brhs, x64, tol, spec_cycles, spec_state, spec_part, d_res,
+                                         st);
         } else {
             if constexpr (std::is_same<R, double>::value)
                 HIPCHK(pcg_solve_plain_fp64(op, brhs, x64, tol, pcg_maxit, pw, d_res, st));
@@ -631,15 +638,15 @@ struct Case : CaseBase {
     }
     int field_solve() override {
         if (int e = solve_x64()) return e;
+        if (spectral) spectral_finish<R>(op, (const R *)brhs, x64, spec_fin, st);
         launch_x_to_phi<R>(G, A_idx, x64, phi, st);
         return 0;
     }
-    // fused step: solve, then phi + voltages + potential in one kernel and E
+    // fused step: solve, then potentials, conductor charge and E in one kernel
     int field_efield_fused() {
         if (int e = solve_x64()) return e;
         mark(1);
-        launch_phi_potential<R>(nc, vc, clk, x64, lap, V, phi, tot, st);
-        launch_efield_only<R>(nc, phi, tot, den, Sigma, Ex, Ey, st);
+        launch_field<R>(nc, vc, clk, op, (const R *)brhs, x64, lap, den, V, phi, tot, Sigma, Ex, Ey, spec_fin, st);
         HIPCHK(hipGetLastError());
         return 0;
     }
@@ -1313,7 +1320,7 @@ struct Case : CaseBase {
         mark(7);
         // deposit + profile sums + id counter and clock advance in one node kernel
         DepositExtras<R> ex{1, sum_den, sum_phi, sum_ex, sum_ey, tot, Ex, Ey, next_id, pstart + G, clk,
-                            (double)S.dt};
+                            (double)S.dt, spec_fin};
         launch_deposit<R>(kc, nc, cur, part, den, sigma_sp, Sigma, Source, brhs, &ex, st);
         if (fluid_on) launch_fluid_step<R>(fl, den, mccr, P1, P2, st);
         HIPCHK(hipGetLastError());
@@ -1825,9 +1832,9 @@ struct Batch : BatchBase {
             if (!c->spectral) return fail(-70, "batch: case %zu does not use the separable field solve", i);
             if (c->timing) return fail(-70, "batch: case %zu has stage timers on", i);
             if (c->fluid_on) return fail(-70, "batch: case %zu runs the metastable fluid", i);
-            if (c->spec_cycles != cs[0]->spec_cycles)
-                return fail(-70, "batch: case %zu's field solve runs %d cycles, case 0's %d", i, c->spec_cycles,
-                            cs[0]->spec_cycles);
+            if (c->spec_kind != cs[0]->spec_kind)
+                return fail(-70, "batch: case %zu's field solve runs %d cycles, case 0's %d", i, c->spec_kind,
+                            cs[0]->spec_kind);
         }
         HIPCHK(hipSetDevice(device));
         HIPCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
@@ -1856,57 +1863,61 @@ struct Batch : BatchBase {
                 rec[q][i] = std::move(r.launches);
             }
         }
-        // lay out the job records and block maps of both parities
-        struct Place { size_t jobs, map; int total; };
+        // at each place of the launch sequence, the cases that run the same
+        // kernel share a grid; lay out its job records and block map
+        struct Place {
+            std::vector<size_t> members;   // cases
+            size_t l, jobs, map;
+            int total;
+        };
+        if (cs.size() >= (1u << (32 - MULTI_LB_BITS))) return fail(-70, "batch: too many cases");
         std::vector<Place> places[2];
         size_t bytes = 0;
         for (int q = 0; q < 2; ++q) {
-            const auto &r0 = rec[q][0];
-            for (size_t i = 1; i < cs.size(); ++i)
-                if (rec[q][i].size() != r0.size()) return fail(-70, "batch: case %zu's step has another launch sequence", i);
-            for (size_t l = 0; l < r0.size(); ++l) {
-                Place pl{};
-                const size_t stride = r0[l].job_size;   // the kernel indexes the records as an array
-                bytes = (bytes + 255) / 256 * 256;
-                pl.jobs = bytes;
-                bytes += stride * cs.size();
-                bytes = (bytes + 255) / 256 * 256;
-                pl.map = bytes;
-                int total = 0;
+            size_t longest = 0;
+            for (const auto &r : rec[q]) longest = std::max(longest, r.size());
+            for (size_t l = 0; l < longest; ++l) {
+                std::vector<bool> placed(cs.size(), false);
                 for (size_t i = 0; i < cs.size(); ++i) {
-                    const RecordedLaunch &x = rec[q][i][l];
-                    if (x.fn != r0[l].fn || x.job_size != r0[l].job_size)
-                        return fail(-70, "batch: case %zu's step has another launch sequence", i);
-                    if (x.blocks >= (1 << MULTI_LB_BITS)) return fail(-70, "batch: a launch of case %zu is too large", i);
-                    total += x.blocks;
+                    if (placed[i] || l >= rec[q][i].size()) continue;
+                    Place pl{};
+                    pl.l = l;
+                    for (size_t k = i; k < cs.size(); ++k) {
+                        if (placed[k] || l >= rec[q][k].size() || rec[q][k][l].fn != rec[q][i][l].fn) continue;
+                        const RecordedLaunch &x = rec[q][k][l];
+                        if (x.blocks >= (1 << MULTI_LB_BITS))
+                            return fail(-70, "batch: a launch of case %zu is too large", k);
+                        placed[k] = true;
+                        pl.members.push_back(k);
+                        pl.total += x.blocks;
+                    }
+                    bytes = (bytes + 255) / 256 * 256;
+                    pl.jobs = bytes;
+                    bytes += rec[q][i][l].job_size * pl.members.size();   // the kernel indexes the records as an array
+                    bytes = (bytes + 255) / 256 * 256;
+                    pl.map = bytes;
+                    bytes += (size_t)pl.total * sizeof(uint32_t);
+                    places[q].push_back(pl);
                 }
-                pl.total = total;
-                bytes += (size_t)total * sizeof(uint32_t);
-                places[q].push_back(pl);
             }
         }
-        if (cs.size() >= (1u << (32 - MULTI_LB_BITS))) return fail(-70, "batch: too many cases");
         std::vector<unsigned char> host(bytes, 0);
         for (int q = 0; q < 2; ++q)
-            for (size_t l = 0; l < places[q].size(); ++l) {
-                const Place &pl = places[q][l];
-                const size_t stride = rec[q][0][l].job_size;
+            for (const Place &pl : places[q]) {
                 uint32_t *map = (uint32_t *)(host.data() + pl.map);
                 int b = 0;
-                for (size_t i = 0; i < cs.size(); ++i) {
-                    const RecordedLaunch &x = rec[q][i][l];
-                    memcpy(host.data() + pl.jobs + i * stride, x.job.data(), x.job_size);
-                    for (int k = 0; k < x.blocks; ++k) map[b++] = ((uint32_t)i << MULTI_LB_BITS) | (uint32_t)k;
+                for (size_t m = 0; m < pl.members.size(); ++m) {
+                    const RecordedLaunch &x = rec[q][pl.members[m]][pl.l];
+                    memcpy(host.data() + pl.jobs + m * x.job_size, x.job.data(), x.job_size);
+                    for (int k = 0; k < x.blocks; ++k) map[b++] = ((uint32_t)m << MULTI_LB_BITS) | (uint32_t)k;
                 }
             }
         HIPCHK(hipMalloc(&dmem, bytes ? bytes : 1));
         HIPCHK(hipMemcpy(dmem, host.data(), bytes, hipMemcpyHostToDevice));
-        for (int q = 0; q < 2; ++q) {
-            for (size_t l = 0; l < places[q].size(); ++l) {
-                const Place &pl = places[q][l];
-                seq[q].push_back(Merged{rec[q][0][l].fn, dmem + pl.jobs, (const uint32_t *)(dmem + pl.map), pl.total});
-            }
-        }
+        for (int q = 0; q < 2; ++q)
+            for (const Place &pl : places[q])
+                seq[q].push_back(Merged{rec[q][pl.members[0]][pl.l].fn, dmem + pl.jobs,
+                                        (const uint32_t *)(dmem + pl.map), pl.total});
         // one graph per parity
         for (int q = 0; q < 2; ++q) {
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));

@@ -16,6 +16,7 @@
 #include "multi.h"
 #include "pic_device.h"
 #include "pic_kernels.h"
+#include "spec_norm.h"
 #include "pic_setup.h"
 
 namespace pic {
@@ -1189,6 +1190,13 @@ __device__ __forceinline__ void deposit_nodes_body(const DepNodesJob<R> &J, int 
     const DepositExtras<R> &ex = J.ex;
 
     int g = bx * blockDim.x + threadIdx.x;
+    if (ex.on && bx == 0 && ex.fin.s && !ex.fin.s->done) {
+        // the field solve's last convergence test, from the partials of k_field
+        __shared__ double sh[2 * RES_BLOCK];
+        double rr, bb;
+        sum_partials(ex.fin.partials, ex.fin.nblk, rr, bb, sh);
+        if (g == 0) spec_decide(rr, bb, ex.fin.tol, 1, ex.fin.s, ex.fin.res);
+    }
     if (ex.on && g == 0) {
         const uint32_t add = (uint32_t)*ex.prod_total_end;
         for (int s = 0; s < n.nsp; ++s) ex.next_id[s] += add;
@@ -1269,54 +1277,6 @@ __global__ __launch_bounds__(256) void k_deposit_nodes_m(const DepNodesJob<R> *J
 }
 
 
-// Fused step: node potential straight from the field solution, with the
-// electrode voltages of this time evaluated per thread:
-// phi = x[A_idx-1] (0 on fixed nodes), tot = sum_c V_c(t) lap_c + phi.
-template <typename R>
-struct PhiPotJob {
-    NodeConst<R> n;
-    VoltConst v;
-    const StepClock *clk;
-    const double *x;
-    const R *lap;
-    R *V, *phi, *tot;
-};
-
-template <typename R>
-__device__ __forceinline__ void phi_potential_body(const PhiPotJob<R> &J, int bx) {
-    const NodeConst<R> &n = J.n;
-    const VoltConst &v = J.v;
-    const StepClock *clk = J.clk;
-    const double *x = J.x;
-    const R *lap = J.lap;
-    R *V = J.V, *phi = J.phi, *tot = J.tot;
-
-    int g = bx * blockDim.x + threadIdx.x;
-    if (g >= n.Gsize) return;
-    const double t = clk->t;
-    const int a = n.A_idx[g];
-    const R ph = a ? (R)x[a - 1] : (R)0;
-    phi[g] = ph;
-    R tp = 0;
-    for (int i = 0; i < n.CondNUMR; ++i) {
-        const R vi = cond_voltage<R>(v, i, t);
-        if (g == 0) V[i] = vi;
-        tp += vi * lap[(size_t)i * n.Gsize + g];
-    }
-    tp += (R)1 * ph;
-    tot[g] = tp;
-}
-
-template <typename R>
-__global__ __launch_bounds__(256) void k_phi_potential(PhiPotJob<R> J) { phi_potential_body<R>(J, blockIdx.x); }
-template <typename R>
-__global__ __launch_bounds__(256) void k_phi_potential_m(const PhiPotJob<R> *J, const uint32_t *map) {
-    int lb;
-    const PhiPotJob<R> &a = J[multi_job(map, lb)];
-    phi_potential_body<R>(a, lb);
-}
-
-
 // ============================================================ EEDF
 // Electron energy histogram: E = Escale v^2 (the MCC's energy, in eV) in
 // EEDF_BINS equal bins over [0, emax); energies at or above emax go to the
@@ -1364,30 +1324,22 @@ __device__ inline void eps_idx(int TID, int ngx, int ngy, int &ET, int &EL, int 
     ET -= (xo + yo); EL -= yo; ED -= xo;
 }
 
+// a node's value and its four neighbours' (its own at the grid's edge)
+template <typename R>
+struct Cross {
+    R c, l, r, d, u;
+};
+
 // Surface charge of conductor/Dirichlet faces (src/cuda_Field.cu:500-558,
 // from the Poisson potential and the last deposit) and node E
 // (src/cuda_Field.cu:698-846, from the total potential).
 template <typename R>
-struct EfieldJob {
-    NodeConst<R> n;
-    const R *phi, *tot, *den;
-    R *Sigma, *Ex, *Ey;
-};
-
-template <typename R>
-__device__ __forceinline__ void efield_body(const EfieldJob<R> &J, int bx) {
-    const NodeConst<R> &n = J.n;
-    const R *phi = J.phi, *tot = J.tot, *den = J.den;
-    R *Sigma = J.Sigma, *Ex = J.Ex, *Ey = J.Ey;
-
-    int TID = bx * blockDim.x + threadIdx.x;
-    if (TID >= n.Gsize) return;
+__device__ __forceinline__ void efield_node(const NodeConst<R> &n, int TID, const Cross<R> &phi, const Cross<R> &Phi,
+                                            const R *den, R *Sigma, R *Ex, R *Ey) {
     const int ngx = n.ngx, ngy = n.ngy;
     const int x = TID / ngy, y = TID % ngy;
     int ET, EL, ED, EC;
     eps_idx<R>(TID, ngx, ngy, ET, EL, ED, EC);
-    const int pl = x ? TID - ngy : TID, pr = (x == ngx - 1) ? TID : TID + ngy;
-    const int pd = y ? TID - 1 : TID, pu = (y == ngy - 1) ? TID : TID + 1;
     const int b = n.Boundary[TID], f = n.Face[TID];
     const R *e = n.eps;
     const R hdx = n.hdx, hdy = n.hdy, idx = n.idx, idy = n.idy, idxy = n.idxy;
@@ -1396,23 +1348,22 @@ __device__ __forceinline__ void efield_body(const EfieldJob<R> &J, int bx) {
     if ((b == CONDUCTOR || b == DIRICHLET) && f != F_NOFACE) {
         R ss = 0;
         for (int i = 0; i < n.nsp; ++i) ss += den[TID + i * n.Gsize] * n.q_density[i];
-        const R P = phi[TID];
+        const R P = phi.c;
         switch (f) {
-        case F_UP: sig = hdy * (e[ET] + e[EL]) * (P - phi[pu]) - hdx * ss; break;
-        case F_DOWN: sig = hdy * (e[ED] + e[EC]) * (P - phi[pd]) - hdx * ss; break;
-        case F_LEFT: sig = hdx * (e[EL] + e[EC]) * (P - phi[pl]) - hdy * ss; break;
-        case F_RIGHT: sig = hdx * (e[ET] + e[ED]) * (P - phi[pr]) - hdy * ss; break;
-        case F_UL: sig = hdy * (e[ET] + e[EL]) * (P - phi[pu]) + hdx * (e[EL] + e[EC]) * (P - phi[pl]) - idxy * ss; break;
-        case F_UR: sig = hdy * (e[ET] + e[EL]) * (P - phi[pu]) + hdx * (e[ET] + e[ED]) * (P - phi[pr]) - idxy * ss; break;
-        case F_LL: sig = hdy * (e[ED] + e[EC]) * (P - phi[pd]) + hdx * (e[EL] + e[EC]) * (P - phi[pl]) - idxy * ss; break;
-        case F_LR: sig = hdy * (e[ED] + e[EC]) * (P - phi[pd]) + hdx * (e[ET] + e[ED]) * (P - phi[pr]) - idxy * ss; break;
+        case F_UP: sig = hdy * (e[ET] + e[EL]) * (P - phi.u) - hdx * ss; break;
+        case F_DOWN: sig = hdy * (e[ED] + e[EC]) * (P - phi.d) - hdx * ss; break;
+        case F_LEFT: sig = hdx * (e[EL] + e[EC]) * (P - phi.l) - hdy * ss; break;
+        case F_RIGHT: sig = hdx * (e[ET] + e[ED]) * (P - phi.r) - hdy * ss; break;
+        case F_UL: sig = hdy * (e[ET] + e[EL]) * (P - phi.u) + hdx * (e[EL] + e[EC]) * (P - phi.l) - idxy * ss; break;
+        case F_UR: sig = hdy * (e[ET] + e[EL]) * (P - phi.u) + hdx * (e[ET] + e[ED]) * (P - phi.r) - idxy * ss; break;
+        case F_LL: sig = hdy * (e[ED] + e[EC]) * (P - phi.d) + hdx * (e[EL] + e[EC]) * (P - phi.l) - idxy * ss; break;
+        case F_LR: sig = hdy * (e[ED] + e[EC]) * (P - phi.d) + hdx * (e[ET] + e[ED]) * (P - phi.r) - idxy * ss; break;
         default: break;
         }
         Sigma[TID] = sig;
     }
     // --- VtoEfield
-    const R *Phi = tot;
-    const R P = Phi[TID];
+    const R P = Phi.c;
     R ex = Ex[TID], ey = Ey[TID];
     const R hxy = n.hxy, hyx = n.hyx;
     const bool wall = (b == CONDUCTOR || b == NEUMANN || b == DIRICHLET);
@@ -1420,74 +1371,166 @@ __device__ __forceinline__ void efield_body(const EfieldJob<R> &J, int bx) {
     const bool hard = (b == CONDUCTOR || b == DIRICHLET || b == DIELECTRIC);
     if (f == F_LEFT) {
         if (wall) { ex = -2 * sig / (e[EL] + e[EC]); ey = 0; }
-        else if (die) { ex = idx * (Phi[pl] - P); ey = hdy * (Phi[pd] - Phi[pu]); }
+        else if (die) { ex = idx * (Phi.l - P); ey = hdy * (Phi.d - Phi.u); }
         else {
-            ex = (R)0.5 * (e[ET] + e[ED]) * (Phi[pr] - P) * idx;
-            ex -= hxy * e[ET] * (P - Phi[pu]) * idy;
-            ex -= hxy * e[ED] * (P - Phi[pd]) * idy;
+            ex = (R)0.5 * (e[ET] + e[ED]) * (Phi.r - P) * idx;
+            ex -= hxy * e[ET] * (P - Phi.u) * idy;
+            ex -= hxy * e[ED] * (P - Phi.d) * idy;
             ex /= (R)-0.5 * (e[EL] + e[EC]);
-            ey = hdy * (Phi[pd] - Phi[pu]);
+            ey = hdy * (Phi.d - Phi.u);
         }
     } else if (f == F_RIGHT) {
         if (wall) { ex = 2 * sig / (e[ET] + e[ED]); ey = 0; }
-        else if (die) { ex = idx * (P - Phi[pr]); ey = hdy * (Phi[pd] - Phi[pu]); }
+        else if (die) { ex = idx * (P - Phi.r); ey = hdy * (Phi.d - Phi.u); }
         else {
-            ex = (R)0.5 * (e[EL] + e[EC]) * (Phi[pl] - P) * idx;
-            ex -= hxy * e[EL] * (P - Phi[pu]) * idy;
-            ex -= hxy * e[EC] * (P - Phi[pd]) * idy;
+            ex = (R)0.5 * (e[EL] + e[EC]) * (Phi.l - P) * idx;
+            ex -= hxy * e[EL] * (P - Phi.u) * idy;
+            ex -= hxy * e[EC] * (P - Phi.d) * idy;
             ex /= (R)0.5 * (e[ET] + e[ED]);
-            ey = hdy * (Phi[pd] - Phi[pu]);
+            ey = hdy * (Phi.d - Phi.u);
         }
     } else if (f == F_UP) {
         if (wall) { ex = 0; ey = 2 * sig / (e[ET] + e[EL]); }
-        else if (die) { ex = hdx * (Phi[pl] - Phi[pr]); ey = idy * (P - Phi[pu]); }
+        else if (die) { ex = hdx * (Phi.l - Phi.r); ey = idy * (P - Phi.u); }
         else {
-            ex = hdx * (Phi[pl] - Phi[pr]);
-            ey = (R)0.5 * (e[ED] + e[EC]) * (Phi[pd] - P) * idy;
-            ey -= hyx * e[ED] * (P - Phi[pr]) * idx;
-            ey -= hyx * e[EC] * (P - Phi[pl]) * idx;
+            ex = hdx * (Phi.l - Phi.r);
+            ey = (R)0.5 * (e[ED] + e[EC]) * (Phi.d - P) * idy;
+            ey -= hyx * e[ED] * (P - Phi.r) * idx;
+            ey -= hyx * e[EC] * (P - Phi.l) * idx;
             ey /= (R)0.5 * (e[ET] + e[EL]);
         }
     } else if (f == F_DOWN) {
         if (wall) { ex = 0; ey = -2 * sig / (e[ED] + e[EC]); }
-        else if (die) { ex = hdx * (Phi[pl] - Phi[pr]); ey = idy * (Phi[pd] - P); }
+        else if (die) { ex = hdx * (Phi.l - Phi.r); ey = idy * (Phi.d - P); }
         else {
-            ex = hdx * (Phi[pl] - Phi[pr]);
-            ey = (R)0.5 * (e[ET] + e[EL]) * (Phi[pu] - P) * idy;
-            ey -= hyx * e[ET] * (P - Phi[pr]) * idx;
-            ey -= hyx * e[EL] * (P - Phi[pl]) * idx;
+            ex = hdx * (Phi.l - Phi.r);
+            ey = (R)0.5 * (e[ET] + e[EL]) * (Phi.u - P) * idy;
+            ey -= hyx * e[ET] * (P - Phi.r) * idx;
+            ey -= hyx * e[EL] * (P - Phi.l) * idx;
             ey /= (R)-0.5 * (e[ED] + e[EC]);
         }
     } else if (f == F_UL) {
-        if (hard) { ex = idx * (Phi[pl] - P); ey = idy * (P - Phi[pu]); }
-        else { ex = hdx * (Phi[pl] - Phi[pr]); ey = hdy * (Phi[pd] - Phi[pu]); }
+        if (hard) { ex = idx * (Phi.l - P); ey = idy * (P - Phi.u); }
+        else { ex = hdx * (Phi.l - Phi.r); ey = hdy * (Phi.d - Phi.u); }
     } else if (f == F_UR) {
-        if (hard) { ex = idx * (P - Phi[pr]); ey = idy * (P - Phi[pu]); }
-        else { ex = hdx * (Phi[pl] - Phi[pr]); ey = hdy * (Phi[pd] - Phi[pu]); }
+        if (hard) { ex = idx * (P - Phi.r); ey = idy * (P - Phi.u); }
+        else { ex = hdx * (Phi.l - Phi.r); ey = hdy * (Phi.d - Phi.u); }
     } else if (f == F_LL) {
-        if (hard) { ex = idx * (Phi[pl] - P); ey = idy * (Phi[pd] - P); }
-        else { ex = hdx * (Phi[pl] - Phi[pr]); ey = hdy * (Phi[pd] - Phi[pu]); }
+        if (hard) { ex = idx * (Phi.l - P); ey = idy * (Phi.d - P); }
+        else { ex = hdx * (Phi.l - Phi.r); ey = hdy * (Phi.d - Phi.u); }
     } else if (f == F_LR) {
-        if (hard) { ex = idx * (P - Phi[pr]); ey = idy * (Phi[pd] - P); }
-        else { ex = hdx * (Phi[pl] - Phi[pr]); ey = hdy * (Phi[pd] - Phi[pu]); }
+        if (hard) { ex = idx * (P - Phi.r); ey = idy * (Phi.d - P); }
+        else { ex = hdx * (Phi.l - Phi.r); ey = hdy * (Phi.d - Phi.u); }
     } else if (b == NEUMANN) {
-        if (x == 0 || x == ngx - 1) { ex = 0; ey = hdy * (Phi[pd] - Phi[pu]); }
-        else if (y == 0 || y == ngy - 1) { ex = hdx * (Phi[pl] - Phi[pr]); ey = 0; }
+        if (x == 0 || x == ngx - 1) { ex = 0; ey = hdy * (Phi.d - Phi.u); }
+        else if (y == 0 || y == ngy - 1) { ex = hdx * (Phi.l - Phi.r); ey = 0; }
     } else {
-        ex = hdx * (Phi[pl] - Phi[pr]);
-        ey = hdy * (Phi[pd] - Phi[pu]);
+        ex = hdx * (Phi.l - Phi.r);
+        ey = hdy * (Phi.d - Phi.u);
     }
     Ex[TID] = ex;
     Ey[TID] = ey;
 }
 
 template <typename R>
-__global__ __launch_bounds__(256) void k_efield(EfieldJob<R> J) { efield_body<R>(J, blockIdx.x); }
+__global__ __launch_bounds__(256) void k_efield(NodeConst<R> n, const R *phi, const R *tot, const R *den, R *Sigma, R *Ex,
+                                                R *Ey) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= n.Gsize) return;
+    const int x = g / n.ngy, y = g % n.ngy;
+    const int l = x ? g - n.ngy : g, r = (x == n.ngx - 1) ? g : g + n.ngy;
+    const int d = y ? g - 1 : g, u = (y == n.ngy - 1) ? g : g + 1;
+    efield_node<R>(n, g, Cross<R>{phi[g], phi[l], phi[r], phi[d], phi[u]},
+                   Cross<R>{tot[g], tot[l], tot[r], tot[d], tot[u]}, den, Sigma, Ex, Ey);
+}
+
+// Fused step: everything between the field solve and the push in one kernel.
+// phi = x[A_idx-1] (0 on fixed nodes), tot = sum_c V_c(t) lap_c + phi, both at
+// the node and, formed again, at its neighbours; then the conductor charge and
+// E.  With F.s the block also sums its unknowns' share of the solve's last
+// residual.  Bound by launch and load latency: as three launches (potential,
+// E, residual) it took 14 us of a 64x64 step, as one 5 us.
 template <typename R>
-__global__ __launch_bounds__(256) void k_efield_m(const EfieldJob<R> *J, const uint32_t *map) {
+struct FieldJob {
+    NodeConst<R> n;
+    VoltConst v;
+    const StepClock *clk;
+    PcgOperator op;
+    const R *b;
+    const double *x;
+    const R *lap, *den;
+    R *V, *phi, *tot, *Sigma, *Ex, *Ey;
+    SpecFinal F;
+};
+
+template <typename R>
+__device__ __forceinline__ void field_body(const FieldJob<R> &J, int bx) {
+    __shared__ R V[MAX_SRC];
+    __shared__ double sh[2 * RES_BLOCK];
+    const NodeConst<R> &n = J.n;
+    const double *xs = J.x;
+    const int g = bx * RES_BLOCK + threadIdx.x;
+    const bool in = g < n.Gsize;
+    const int gc = in ? g : 0;
+    const int x = gc / n.ngy, y = gc % n.ngy;
+    const int at[5] = {gc, x ? gc - n.ngy : gc, (x == n.ngx - 1) ? gc : gc + n.ngy, y ? gc - 1 : gc,
+                       (y == n.ngy - 1) ? gc : gc + 1};
+    int a[5];
+    R ph[5], tp[5];
+    // the loads first: they are in flight while the first threads form the voltages
+#pragma unroll
+    for (int k = 0; k < 5; ++k) a[k] = n.A_idx[at[k]];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        ph[k] = a[k] ? (R)xs[a[k] - 1] : (R)0;
+        tp[k] = 0;
+    }
+    if ((int)threadIdx.x < n.CondNUMR) {
+        const R vi = cond_voltage<R>(J.v, threadIdx.x, J.clk->t);
+        V[threadIdx.x] = vi;
+        if (bx == 0) J.V[threadIdx.x] = vi;
+    }
+    __syncthreads();
+    double rr = 0.0, bb = 0.0;
+    if (in) {
+        for (int i = 0; i < n.CondNUMR; ++i) {
+            const R *lap = J.lap + (size_t)i * n.Gsize;
+#pragma unroll
+            for (int k = 0; k < 5; ++k) tp[k] += V[i] * lap[at[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < 5; ++k) tp[k] += (R)1 * ph[k];
+        J.phi[g] = ph[0];
+        J.tot[g] = tp[0];
+        efield_node<R>(n, g, Cross<R>{ph[0], ph[1], ph[2], ph[3], ph[4]}, Cross<R>{tp[0], tp[1], tp[2], tp[3], tp[4]},
+                       J.den, J.Sigma, J.Ex, J.Ey);
+        if (J.F.s && a[0]) {
+            const int o = 5 * (a[0] - 1);
+            double ax = J.op.vald[o] * xs[J.op.col[o]];
+#pragma unroll
+            for (int e = 1; e < 5; ++e) ax += J.op.vald[o + e] * xs[J.op.col[o + e]];
+            const double bi = (double)J.b[a[0] - 1], ri = bi - ax;
+            rr = ri * ri;
+            bb = bi * bi;
+        }
+    }
+    if (J.F.s) {
+        block_sum2<RES_BLOCK>(rr, bb, sh);
+        if (threadIdx.x == 0) {
+            double *part = const_cast<double *>(J.F.partials);
+            part[2 * bx] = rr;
+            part[2 * bx + 1] = bb;
+        }
+    }
+}
+
+template <typename R>
+__global__ __launch_bounds__(RES_BLOCK) void k_field(FieldJob<R> J) { field_body<R>(J, blockIdx.x); }
+template <typename R>
+__global__ __launch_bounds__(RES_BLOCK) void k_field_m(const FieldJob<R> *J, const uint32_t *map) {
     int lb;
-    const EfieldJob<R> &a = J[multi_job(map, lb)];
-    efield_body<R>(a, lb);
+    const FieldJob<R> &a = J[multi_job(map, lb)];
+    field_body<R>(a, lb);
 }
 
 
@@ -1646,33 +1689,26 @@ template <typename R>
 void launch_eedf(const PView<R> &p, int Gsize, R escale, R emax, unsigned long long *hist, hipStream_t s) {
     hipLaunchKernelGGL(k_eedf<R>, dim3(1024), dim3(256), 0, s, p, Gsize, escale, emax, hist);
 }
+int field_partials(int Gsize) { return (Gsize + RES_BLOCK - 1) / RES_BLOCK; }
 template <typename R>
-void launch_phi_potential(const NodeConst<R> &n, const VoltConst &v, const StepClock *clk, const double *x,
-                          const R *lap, R *V, R *phi, R *tot, hipStream_t s) {
-    const PhiPotJob<R> J{n, v, clk, x, lap, V, phi, tot};
+void launch_field(const NodeConst<R> &n, const VoltConst &v, const StepClock *clk, const PcgOperator &op, const R *b,
+                  const double *x, const R *lap, const R *den, R *V, R *phi, R *tot, R *Sigma, R *Ex, R *Ey,
+                  SpecFinal &F, hipStream_t s) {
+    F.nblk = field_partials(n.Gsize);
+    const FieldJob<R> J{n, v, clk, op, b, x, lap, den, V, phi, tot, Sigma, Ex, Ey, F};
     if (Recorder *r = launch_recorder()) {
-        r->add(&launch_m<PhiPotJob<R>, k_phi_potential_m<R>, 256>, J, node_blocks(n.Gsize));
+        r->add(&launch_m<FieldJob<R>, k_field_m<R>, RES_BLOCK>, J, F.nblk);
         return;
     }
-    hipLaunchKernelGGL(k_phi_potential<R>, dim3(node_blocks(n.Gsize)), dim3(256), 0, s, J);
-}
-template <typename R>
-void launch_efield_only(const NodeConst<R> &n, const R *phi, const R *tot, const R *den, R *Sigma, R *Ex, R *Ey,
-                        hipStream_t s) {
-    const EfieldJob<R> J{n, phi, tot, den, Sigma, Ex, Ey};
-    if (Recorder *r = launch_recorder()) {
-        r->add(&launch_m<EfieldJob<R>, k_efield_m<R>, 256>, J, node_blocks(n.Gsize));
-        return;
-    }
-    hipLaunchKernelGGL(k_efield<R>, dim3(node_blocks(n.Gsize)), dim3(256), 0, s, J);
+    hipLaunchKernelGGL(k_field<R>, dim3(F.nblk), dim3(RES_BLOCK), 0, s, J);
 }
 template <typename R>
 void launch_efield(const NodeConst<R> &n, const VoltConst &v, double t, const R *lap, R *V, const R *phi, R *tot,
                    const R *den, R *Sigma, R *Ex, R *Ey, hipStream_t s) {
     hipLaunchKernelGGL(k_voltages<R>, dim3(1), dim3(64), 0, s, v, t, V);
     hipLaunchKernelGGL(k_potential<R>, dim3(node_blocks(n.Gsize)), dim3(256), 0, s, n, lap, (const R *)V, phi, tot);
-    hipLaunchKernelGGL(k_efield<R>, dim3(node_blocks(n.Gsize)), dim3(256), 0, s,
-                       EfieldJob<R>{n, phi, (const R *)tot, den, Sigma, Ex, Ey});
+    hipLaunchKernelGGL(k_efield<R>, dim3(node_blocks(n.Gsize)), dim3(256), 0, s, n, phi, (const R *)tot, den, Sigma, Ex,
+                       Ey);
 }
 template <typename R>
 void launch_accumulate(int Gsize, int nsp, const R *den, const R *tot, const R *Ex, const R *Ey, double *sden,
@@ -1699,7 +1735,6 @@ void launch_x_to_phi(int Gsize, const int *A_idx, const double *x, R *phi, hipSt
     hipLaunchKernelGGL(k_x_to_phi<R>, dim3(node_blocks(Gsize)), dim3(256), 0, s, Gsize, A_idx, x, phi);
 }
 template void launch_rhs_to_fp64<float>(int, const float *, double *, hipStream_t);
-template void launch_rhs_to_fp64<double>(int, const double *, double *, hipStream_t);
 template void launch_x_to_phi<float>(int, const int *, const double *, float *, hipStream_t);
 template void launch_x_to_phi<double>(int, const int *, const double *, double *, hipStream_t);
 
@@ -1776,11 +1811,10 @@ void launch_scan(const int *in, int *out, int n, int *tmp, hipStream_t s) {
                                           const int *, const int *, const uint32_t *, int, int, int *, hipStream_t);   \
     template void launch_deposit<R>(const DevConst<R> &, const NodeConst<R> &, const PView<R> *, R *, R *, R *, R *,   \
                                     R *, R *, const DepositExtras<R> *, hipStream_t);                                  \
-    template void launch_phi_potential<R>(const NodeConst<R> &, const VoltConst &, const StepClock *, const double *,  \
-                                          const R *, R *, R *, R *, hipStream_t);                                      \
     template void launch_eedf<R>(const PView<R> &, int, R, R, unsigned long long *, hipStream_t);               \
-    template void launch_efield_only<R>(const NodeConst<R> &, const R *, const R *, const R *, R *, R *, R *,          \
-                                        hipStream_t);                                                            \
+    template void launch_field<R>(const NodeConst<R> &, const VoltConst &, const StepClock *, const PcgOperator &,    \
+                                  const R *, const double *, const R *, const R *, R *, R *, R *, R *, R *, R *,       \
+                                  SpecFinal &, hipStream_t);                                                           \
     template void launch_efield<R>(const NodeConst<R> &, const VoltConst &, double, const R *, R *, const R *, R *,    \
                                    const R *, R *, R *, R *, hipStream_t);                                             \
     template void launch_accumulate<R>(int, int, const R *, const R *, const R *, const R *, double *, double *,       \

@@ -4,7 +4,8 @@
 // for all of them: the launches a case's step would make are recorded (the
 // kernel's merged-grid launcher, its argument record and its block count),
 // the records of the same launch of every case are placed side by side in
-// device memory, and one grid covers all their blocks.  Block b of that grid
+// device memory, and one grid covers all their blocks (cases whose step runs
+// another kernel at that place of the sequence get a grid of their own).  Block b of that grid
 // reads map[b] = job << MULTI_LB_BITS | block-within-job, and runs the
 // kernel's body with that job's arguments as that block.
 #pragma once

@@ -68,6 +68,41 @@ struct StepClock {
     double t;
 };
 
+// Operator in padded 5-entry row form (missing entries have col = row, val = 0).
+struct PcgOperator {
+    int N;
+    const int *col;          // 5N
+    const float *valf;       // 5N
+    const double *vald;      // 5N
+    const float *mdiagf;     // N   Jacobi preconditioner 1/diag
+    const double *mdiagd;
+};
+
+// ---- separable field solve (spectral.hip): device tables and state
+struct PcgResult {
+    int iters;          // total inner iterations
+    int outer;          // refinement cycles (1 for the plain path)
+    double rel_res;     // final ||b - A x|| / ||b|| in FP64
+    int status;         // 0 converged, 1 hit the iteration limit, 3 abandoned (a grid barrier wait timed out)
+};
+struct SpecDev {
+    int nx, ny;
+    const double *Vxi, *VyiT, *Vx, *VyT, *dinv;     // dinv = 1/(cx lx_a + cy ly_b + shift), 0 for a null mode
+    double *T1, *T2, *r;                            // nx*ny work matrices, r = residual
+};
+struct SpecState {
+    int done, outer, status, pad;
+    double rel;
+};
+// what the convergence test after a cycle needs
+struct SpecFinal {
+    const double *partials;   // nblk pairs of ||r||^2, ||b||^2
+    int nblk;
+    double tol;
+    SpecState *s;             // null: nothing to decide
+    PcgResult *res;
+};
+
 // fused-step extras of the node deposit kernel: FP64 profile sums, the
 // particle id counters (advanced by the step's product count) and the clock
 template <typename R>
@@ -79,6 +114,7 @@ struct DepositExtras {
     const int *prod_total_end;
     StepClock *clk;
     double dt;
+    SpecFinal fin;   // the field solve's last convergence test
 };
 
 constexpr int MAX_SRC = 16;
@@ -129,16 +165,17 @@ void launch_fused_scatter(const DevConst<R> &, const PView<R> &p, const PView<R>
 template <typename R>
 void launch_deposit(const DevConst<R> &, const NodeConst<R> &, const PView<R> *, R *part, R *den, R *sigma_sp,
                     R *Sigma, R *Source, R *b, const DepositExtras<R> *ex, hipStream_t);
-// fused step: phi from the FP64 solution, electrode voltages and total potential in one kernel
+// fused step: phi from the FP64 solution, electrode voltages, total potential,
+// conductor charge and E, and with F.s the partial norms of the solve's last
+// residual (op, b), all in one kernel.  F.nblk becomes the number of partials.
 template <typename R>
-void launch_phi_potential(const NodeConst<R> &n, const VoltConst &v, const StepClock *clk, const double *x,
-                          const R *lap, R *V, R *phi, R *tot, hipStream_t s);
+void launch_field(const NodeConst<R> &n, const VoltConst &v, const StepClock *clk, const PcgOperator &op, const R *b,
+                  const double *x, const R *lap, const R *den, R *V, R *phi, R *tot, R *Sigma, R *Ex, R *Ey,
+                  SpecFinal &F, hipStream_t s);
+int field_partials(int Gsize);   // pairs launch_field writes
 // electron energy histogram (EEDF_BINS bins over [0, emax) eV) added into hist
 template <typename R>
 void launch_eedf(const PView<R> &electrons, int Gsize, R escale, R emax, unsigned long long *hist, hipStream_t s);
-template <typename R>
-void launch_efield_only(const NodeConst<R> &n, const R *phi, const R *tot, const R *den, R *Sigma, R *Ex, R *Ey,
-                        hipStream_t s);
 template <typename R>
 void launch_efield(const NodeConst<R> &, const VoltConst &, double, const R *, R *, const R *, R *, const R *, R *, R *,
                    R *, hipStream_t);
@@ -177,23 +214,6 @@ template <typename R> void launch_rhs_to_fp64(int N, const R *b, double *b64, hi
 template <typename R> void launch_x_to_phi(int Gsize, const int *A_idx, const double *x, R *phi, hipStream_t s);
 
 // ---- field solver (pcg.hip)
-struct PcgResult {
-    int iters;          // total inner iterations
-    int outer;          // refinement cycles (1 for the plain path)
-    double rel_res;     // final ||b - A x|| / ||b|| in FP64
-    int status;         // 0 converged, 1 hit the iteration limit, 3 abandoned (a grid barrier wait timed out)
-};
-
-// Operator in padded 5-entry row form (missing entries have col = row, val = 0).
-struct PcgOperator {
-    int N;
-    const int *col;          // 5N
-    const float *valf;       // 5N
-    const double *vald;      // 5N
-    const float *mdiagf;     // N   Jacobi preconditioner 1/diag
-    const double *mdiagd;
-};
-
 struct PcgWork;   // device scratch owned by the context
 // col, val: the operator's 5N columns and values (host)
 PcgWork *pcg_work_create(int N, const int *col, const double *val, int *err, int want_blocks, hipStream_t stream);
@@ -249,19 +269,13 @@ hipError_t pcg_solve_refined(const PcgOperator &A, const float *b, double *b64, 
                              double inner_tol, int maxit, PcgWork *w, PcgResult *res, hipStream_t s);
 
 // ---- separable fast solve (spectral.hip), FP64 throughout
-struct SpecDev {
-    int nx, ny;
-    const double *Vxi, *VyiT, *Vx, *VyT, *dinv;   // dinv = 1/(cx lx_a + cy ly_b), 0 for a null mode
-    double *T1, *T2, *r;                            // nx*ny work matrices, r = residual
-};
-struct SpecState {
-    int done, outer, status, pad;
-    double rel;
-};
-// b32 = right-hand side (FP32 or FP64), converted into b (FP64) by the first residual
+// enqueues max_cycles refinement cycles on x; the convergence test after the
+// last one is left to the caller: spectral_finish, or the fused step's later
+// kernels through the returned record
 template <typename RB>
-void spectral_solve_refined(const PcgOperator &A, const SpecDev &sp, const RB *b32, double *b, double *x,
-                            double tol, int max_cycles, SpecState *state, double *partials, PcgResult *res,
-                            hipStream_t st);
+SpecFinal spectral_solve(const PcgOperator &A, const SpecDev &sp, const RB *b, double *x, double tol, int max_cycles,
+                         SpecState *state, double *partials, PcgResult *res, hipStream_t st);
+template <typename RB>
+void spectral_finish(const PcgOperator &A, const RB *b, const double *x, const SpecFinal &F, hipStream_t st);
 
 }  // namespace pic

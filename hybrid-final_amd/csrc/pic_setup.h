@@ -113,8 +113,9 @@ int build_setup(const Deck &d, Setup<R> &s, std::string &err, bool load = true);
 struct Spectral {
     bool ok = false;
     bool exact = false;   // every operator entry equals the separable model bit for bit
+    bool shifted = false; // ... with a non-zero shift
     int nx = 0, ny = 0;
-    double cx = 0, cy = 0;
+    double cx = 0, cy = 0, shift = 0;
     std::vector<double> Vx, Vxi, Vy, Vyi, lx, ly;
 };
 template <typename R>
