@@ -1288,10 +1288,18 @@ struct Case : CaseBase {
         // ionisation stash reuses its product staging buffer (stride = the
         // largest capacity)
         const size_t sstride = (size_t)stage_stride;
-        launch_fused_count<R>(kc, cur[0], 0, clk, cnt[0], pcnt, mccr, condcharge, tag[0], stage, sstride, d_err, st);
+        const bool pair = !timing;   // the stage timers tell the species apart
+        auto count = [&](int which) {
+            launch_fused_count<R>(kc, cur[0], cur[1], which, clk, cnt[0], cnt[1], pcnt, mccr, condcharge, tag[0],
+                                  tag[1], stage, sstride, d_err, st);
+        };
+        auto scatter = [&](int which) {
+            launch_fused_scatter<R>(kc, cur[0], cur[1], nxt[0], nxt[1], which, tag[0], tag[1], stage, sstride, base[0],
+                                    base[1], pbase[0], pbase[1], pid_off, next_id, d_err, st);
+        };
+        count(pair ? 2 : 0);
         mark(3);
-        launch_fused_count<R>(kc, cur[1], 1, clk, cnt[1], nullptr, mccr, condcharge, tag[1], stage, sstride, d_err,
-                              st);
+        if (!pair) count(1);
         mark(4);
         // survivors + ionisation products per destination cell for both
         // species, their three scans (electron and ion cell_start, global
@@ -1300,11 +1308,9 @@ struct Case : CaseBase {
                           nxt[0].cell_start, nxt[1].cell_start, pstart, base[0], base[1], pbase[0], pbase[1], pid_off,
                           scan_tmp, st);
         mark(5);
-        launch_fused_scatter<R>(kc, cur[0], nxt[0], nxt[1], 0, tag[0], stage, sstride, base[0], pbase[0], pbase[1],
-                                pid_off, next_id, nxt[0].cap, nxt[1].cap, d_err, st);
+        scatter(pair ? 2 : 0);
         mark(6);
-        launch_fused_scatter<R>(kc, cur[1], nxt[1], nxt[1], 1, tag[1], stage, sstride, base[1], pbase[1], pbase[1],
-                                pid_off, next_id, nxt[1].cap, nxt[1].cap, d_err, st);
+        if (!pair) scatter(1);
         // the id counters advance in the deposit that follows (after both scatters)
         swap_species(0);
         swap_species(1);
@@ -1856,6 +1862,7 @@ struct Batch : BatchBase {
                 }
                 expect[q].push_back(c->cur[0].x);
                 Recorder r;
+                for (auto *o : cs) r.cells += o->S.Csize;
                 launch_recorder() = &r;
                 const int e = c->enqueue_step();
                 launch_recorder() = nullptr;

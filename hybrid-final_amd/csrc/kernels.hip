@@ -28,6 +28,13 @@ Recorder *&launch_recorder() {
 
 namespace {
 
+// a particle view with its pointers known as device memory
+template <typename R>
+__device__ inline PView<R> device_view(const PView<R> &p) {
+    return PView<R>{device_ptr(p.x), device_ptr(p.y), device_ptr(p.vx), device_ptr(p.vy), device_ptr(p.vz),
+                    device_ptr(p.id), device_ptr(p.cell_start), p.cap};
+}
+
 template <typename R>
 __device__ inline R wave_sum(R v) {
 #pragma unroll
@@ -393,7 +400,7 @@ __device__ __forceinline__ void pair_totals_body(const PairTotalsJob &J, int bx)
 __global__ __launch_bounds__(BASES_TILE) void k_pair_totals(PairTotalsJob J) { pair_totals_body(J, blockIdx.x); }
 __global__ __launch_bounds__(BASES_TILE) void k_pair_totals_m(const PairTotalsJob *J, const uint32_t *map) {
     int lb;
-    const PairTotalsJob &a = J[multi_job(map, lb)];
+    const PairTotalsJob &a = multi_record(J, map, lb);
     pair_totals_body(a, lb);
 }
 
@@ -481,7 +488,7 @@ __device__ __forceinline__ void pair_scan_bases_body(const PairBasesJob &J, int 
 __global__ __launch_bounds__(BASES_TILE) void k_pair_scan_bases(PairBasesJob J) { pair_scan_bases_body(J, blockIdx.x); }
 __global__ __launch_bounds__(BASES_TILE) void k_pair_scan_bases_m(const PairBasesJob *J, const uint32_t *map) {
     int lb;
-    const PairBasesJob &a = J[multi_job(map, lb)];
+    const PairBasesJob &a = multi_record(J, map, lb);
     pair_scan_bases_body(a, lb);
 }
 
@@ -738,10 +745,15 @@ __device__ inline int collide(const DevConst<R> &k, int dest, R pa, uint32_t id,
 // LDS queue with their post-push state, and whenever 64 are queued they
 // collide together, one per lane, so the long collision code runs on full
 // wavefronts.  The waves of a block never wait for each other.
-constexpr int CPW = 4;          // cells per wave (at most 16: the queue keeps the cell in 4 bits)
+// CPW, the cells per wave (at most 16: the queue keeps the cell in 4 bits), is
+// 4 where that still makes 4096 waves, 16 to a CU: below, one wave's chain of
+// tables, walk and collisions is what a step waits for (64x64: 105 us per step
+// with four cells per wave from 8192 cells on down to 93 with one; 100x100: 130
+// and 118; above 16384 cells all choices are within 2 %).
+constexpr int COUNT_WIDE = 16384;
 constexpr int CQCAP = 128;      // queued colliders per wave (< 64 left after each collide, + 64 per walk step)
 
-template <typename R>
+template <typename R, int CPW>
 struct CountWave {
     // collider queue: post-push state, particle index and (draw << 8 | cell << 4 | move code)
     R qx[CQCAP], qy[CQCAP], qvx[CQCAP], qvy[CQCAP], qvz[CQCAP];
@@ -769,20 +781,20 @@ struct CountJob {
     int *err;
 };
 
-template <typename R, int KIND>
-__device__ __forceinline__ void fused_count_body(const CountJob<R> &J, int bx) {
+template <typename R, int KIND, int CPW>
+__device__ __forceinline__ void fused_count_body(const CountJob<R> &J, int bx, CountWave<R, CPW> *waves) {
     const DevConst<R> &k = J.k;
-    const PView<R> &p = J.p;
+    const PView<R> p = device_view(J.p);
     const int isp = J.isp;
-    const StepClock *clk = J.clk;
-    int *cnt = J.cnt, *pcnt = J.pcnt, *condcharge = J.condcharge, *err = J.err;
-    unsigned long long *mccr = J.mccr;
-    uint8_t *flag = J.flag;
-    R *stash = J.stash;
+    const StepClock *clk = device_ptr(J.clk);
+    int *cnt = device_ptr(J.cnt), *pcnt = device_ptr(J.pcnt), *condcharge = device_ptr(J.condcharge),
+        *err = device_ptr(J.err);
+    unsigned long long *mccr = device_ptr(J.mccr);
+    uint8_t *flag = device_ptr(J.flag);
+    R *stash = device_ptr(J.stash);
     const size_t stash_stride = J.stash_stride;
 
-    __shared__ CountWave<R> waves[FWAVES];
-    CountWave<R> &W = waves[threadIdx.x >> 6];
+    CountWave<R, CPW> &W = waves[threadIdx.x >> 6];
     const uint32_t step = clk->step;
     const int lane = threadIdx.x & 63;
     const int w0 = __builtin_amdgcn_readfirstlane((int)((bx * blockDim.x + threadIdx.x) >> 6)) * CPW;
@@ -807,6 +819,14 @@ __device__ __forceinline__ void fused_count_body(const CountJob<R> &J, int bx) {
         }
     }
     const int hi = lo[CPW];
+    // the first particles, in flight while the tables are made; lanes past
+    // the end reload the last particle (never used)
+    R x = 0, y = 0, vx = 0, vy = 0, vz = 0;
+    uint32_t id = 0;
+    if (lo[0] < hi) {
+        const int i = min(lo[0] + lane, hi - 1);
+        x = p.x[i]; y = p.y[i]; vx = p.vx[i]; vy = p.vy[i]; vz = p.vz[i]; id = p.id[i];
+    }
     // per-wave tables
     for (int t = lane; t < CPW * ROUTE_SLOTS; t += 64) {
         const int q = t / ROUTE_SLOTS;
@@ -867,14 +887,7 @@ __device__ __forceinline__ void fused_count_body(const CountJob<R> &J, int bx) {
         }
     };
 
-    // the walk, 64 particles at a time; lanes past the end reload the last
-    // particle (never used)
-    R x = 0, y = 0, vx = 0, vy = 0, vz = 0;
-    uint32_t id = 0;
-    if (lo[0] < hi) {
-        const int i = min(lo[0] + lane, hi - 1);
-        x = p.x[i]; y = p.y[i]; vx = p.vx[i]; vy = p.vy[i]; vz = p.vz[i]; id = p.id[i];
-    }
+    // the walk, 64 particles at a time
     for (int b = lo[0]; b < hi; b += 64) {
         R nx = 0, ny = 0, nvx = 0, nvy = 0, nvz = 0;
         uint32_t nid = 0;
@@ -956,13 +969,41 @@ __device__ __forceinline__ void fused_count_body(const CountJob<R> &J, int bx) {
     }
 }
 
-template <typename R, int KIND>
-__global__ __launch_bounds__(256) void k_fused_count(CountJob<R> J) { fused_count_body<R, KIND>(J, blockIdx.x); }
-template <typename R, int KIND>
+template <typename R, int KIND, int CPW>
+__global__ __launch_bounds__(256) void k_fused_count(CountJob<R> J) {
+    __shared__ CountWave<R, CPW> waves[FWAVES];
+    fused_count_body<R, KIND, CPW>(J, blockIdx.x, waves);
+}
+template <typename R, int KIND, int CPW>
 __global__ __launch_bounds__(256) void k_fused_count_m(const CountJob<R> *J, const uint32_t *map) {
+    __shared__ CountWave<R, CPW> waves[FWAVES];
     int lb;
-    const CountJob<R> &a = J[multi_job(map, lb)];
-    fused_count_body<R, KIND>(a, lb);
+    const CountJob<R> &a = multi_record(J, map, lb);
+    fused_count_body<R, KIND, CPW>(a, lb, waves);
+}
+// both species in one launch, blocks [0, nb) electrons, [nb, 2 nb) ions: the
+// ions fill the chip while the last electron blocks finish.  Both passes
+// together, against a launch per species, us per step: 64x64 93 against 105,
+// 75x181 134 against 158, 128x128 145 against 169, 256x256 at 200 particles per
+// cell 801 against 825.  (Blocks of the two species interleaved were slower.)
+template <typename R>
+struct CountPair {
+    CountJob<R> e, i;
+    int nb;
+};
+template <typename R, int CPW>
+__device__ __forceinline__ void fused_count_pair(const CountPair<R> &J, int bx) {
+    __shared__ CountWave<R, CPW> waves[FWAVES];
+    if (bx < J.nb) fused_count_body<R, KIND_AR_ELECTRON, CPW>(J.e, bx, waves);
+    else fused_count_body<R, KIND_AR_ION, CPW>(J.i, bx - J.nb, waves);
+}
+template <typename R, int CPW>
+__global__ __launch_bounds__(256) void k_fused_count2(CountPair<R> J) { fused_count_pair<R, CPW>(J, blockIdx.x); }
+template <typename R, int CPW>
+__global__ __launch_bounds__(256) void k_fused_count2_m(const CountPair<R> *J, const uint32_t *map) {
+    int lb;
+    const CountPair<R> &a = multi_record(J, map, lb);
+    fused_count_pair<R, CPW>(a, lb);
 }
 
 
@@ -985,28 +1026,33 @@ struct ScatterJob {
     int *err;
 };
 
-template <typename R, int KIND>
-__device__ __forceinline__ void fused_scatter_body(const ScatterJob<R> &J, int bx) {
-    const DevConst<R> &k = J.k;
-    const PView<R> &p = J.p, &q = J.q, &qion = J.qion;
-    const int isp = J.isp, cap = J.cap, cap_ion = J.cap_ion;
-    const uint8_t *flag = J.flag;
-    const R *stash = J.stash;
-    const size_t stash_stride = J.stash_stride;
-    const int *base = J.base, *pbase_e = J.pbase_e, *pbase_i = J.pbase_i, *pid_off = J.pid_off;
-    const uint32_t *next_id = J.next_id;
-    int *err = J.err;
+template <typename R>
+struct ScatterLds {
+    FStage<R, SCHUNK> stage[FWAVES];
+    uint8_t flag[FWAVES][SCHUNK];
+};
 
-    __shared__ FStage<R, SCHUNK> stage_all[FWAVES];
-    __shared__ uint8_t flag_all[FWAVES][SCHUNK];
+template <typename R, int KIND>
+__device__ __forceinline__ void fused_scatter_body(const ScatterJob<R> &J, int bx, ScatterLds<R> &lds) {
+    const DevConst<R> &k = J.k;
+    const PView<R> p = device_view(J.p), q = device_view(J.q), qion = device_view(J.qion);
+    const int isp = J.isp, cap = J.cap, cap_ion = J.cap_ion;
+    const uint8_t *flag = device_ptr(J.flag);
+    const R *stash = device_ptr(J.stash);
+    const size_t stash_stride = J.stash_stride;
+    const int *base = device_ptr(J.base), *pbase_e = device_ptr(J.pbase_e), *pbase_i = device_ptr(J.pbase_i),
+              *pid_off = device_ptr(J.pid_off);
+    const uint32_t *next_id = device_ptr(J.next_id);
+    int *err = device_ptr(J.err);
+
     int lane;
     int c = wave_cell_b(k.ncy, k.ngy, k.Csize, lane, bx);
     if (c < 0) return;
     int k0, k1;
     cell_range(p, c, k0, k1);
     if (k0 == k1) return;
-    FStage<R, SCHUNK> &S = stage_all[threadIdx.x >> 6];
-    uint8_t *F = flag_all[threadIdx.x >> 6];
+    FStage<R, SCHUNK> &S = lds.stage[threadIdx.x >> 6];
+    uint8_t *F = lds.flag[threadIdx.x >> 6];
     CellE<R> e;
     e.load(k.Ex, k.Ey, c, k.ngy);
     const Route myr = lane < ROUTE_SLOTS ? k.route[c * ROUTE_SLOTS + lane] : Route{-1, 0};
@@ -1092,12 +1138,36 @@ __device__ __forceinline__ void fused_scatter_body(const ScatterJob<R> &J, int b
 }
 
 template <typename R, int KIND>
-__global__ __launch_bounds__(256) void k_fused_scatter(ScatterJob<R> J) { fused_scatter_body<R, KIND>(J, blockIdx.x); }
+__global__ __launch_bounds__(256) void k_fused_scatter(ScatterJob<R> J) {
+    __shared__ ScatterLds<R> lds;
+    fused_scatter_body<R, KIND>(J, blockIdx.x, lds);
+}
 template <typename R, int KIND>
 __global__ __launch_bounds__(256) void k_fused_scatter_m(const ScatterJob<R> *J, const uint32_t *map) {
+    __shared__ ScatterLds<R> lds;
     int lb;
-    const ScatterJob<R> &a = J[multi_job(map, lb)];
-    fused_scatter_body<R, KIND>(a, lb);
+    const ScatterJob<R> &a = multi_record(J, map, lb);
+    fused_scatter_body<R, KIND>(a, lb, lds);
+}
+// both species in one launch, as in the count pass
+template <typename R>
+struct ScatterPair {
+    ScatterJob<R> e, i;
+    int nb;
+};
+template <typename R>
+__device__ __forceinline__ void fused_scatter_pair(const ScatterPair<R> &J, int bx) {
+    __shared__ ScatterLds<R> lds;
+    if (bx < J.nb) fused_scatter_body<R, KIND_AR_ELECTRON>(J.e, bx, lds);
+    else fused_scatter_body<R, KIND_AR_ION>(J.i, bx - J.nb, lds);
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_fused_scatter2(ScatterPair<R> J) { fused_scatter_pair<R>(J, blockIdx.x); }
+template <typename R>
+__global__ __launch_bounds__(256) void k_fused_scatter2_m(const ScatterPair<R> *J, const uint32_t *map) {
+    int lb;
+    const ScatterPair<R> &a = multi_record(J, map, lb);
+    fused_scatter_pair<R>(a, lb);
 }
 
 
@@ -1161,7 +1231,7 @@ __global__ __launch_bounds__(256) void k_deposit_cells(DepCellsJob<R> J) {
 template <typename R>
 __global__ __launch_bounds__(256) void k_deposit_cells_m(const DepCellsJob<R> *J, const uint32_t *map) {
     int lb;
-    const DepCellsJob<R> &a = J[multi_job(map, lb)];
+    const DepCellsJob<R> &a = multi_record(J, map, lb);
     deposit_cells_body<R>(a, lb % a.gx, lb / a.gx);
 }
 
@@ -1272,7 +1342,7 @@ __global__ __launch_bounds__(256) void k_deposit_nodes(DepNodesJob<R> J) { depos
 template <typename R>
 __global__ __launch_bounds__(256) void k_deposit_nodes_m(const DepNodesJob<R> *J, const uint32_t *map) {
     int lb;
-    const DepNodesJob<R> &a = J[multi_job(map, lb)];
+    const DepNodesJob<R> &a = multi_record(J, map, lb);
     deposit_nodes_body<R>(a, lb);
 }
 
@@ -1529,7 +1599,7 @@ __global__ __launch_bounds__(RES_BLOCK) void k_field(FieldJob<R> J) { field_body
 template <typename R>
 __global__ __launch_bounds__(RES_BLOCK) void k_field_m(const FieldJob<R> *J, const uint32_t *map) {
     int lb;
-    const FieldJob<R> &a = J[multi_job(map, lb)];
+    const FieldJob<R> &a = multi_record(J, map, lb);
     field_body<R>(a, lb);
 }
 
@@ -1593,8 +1663,13 @@ __global__ void k_x_to_phi(int Gsize, const int *A_idx, const double *x, R *phi)
 
 // ============================================================ launchers
 static inline int cell_blocks(int Csize) { return (Csize + 3) / 4; }
-// count pass: CPW cells per wave, FWAVES waves per block
-static inline int count_blocks(int Csize) { return (Csize + CPW * FWAVES - 1) / (CPW * FWAVES); }
+// count pass: cells per wave and blocks (FWAVES waves per block)
+static inline long long grid_cells(int Csize) { return launch_recorder() ? launch_recorder()->cells : Csize; }
+static inline int count_cpw(int Csize) {
+    const long long n = grid_cells(Csize);
+    return n >= COUNT_WIDE ? 4 : n >= COUNT_WIDE / 2 ? 2 : 1;
+}
+static inline int count_blocks(int Csize, int cpw) { return (Csize + cpw * FWAVES - 1) / (cpw * FWAVES); }
 static inline int node_blocks(int n) { return (n + 255) / 256; }
 
 template <typename R>
@@ -1632,41 +1707,44 @@ void launch_mcc_insert(const DevConst<R> &k, const PView<R> &src, const PView<R>
     hipLaunchKernelGGL(k_mcc_insert<R>, dim3(cell_blocks(k.Csize)), dim3(256), 0, s, k, src, dst, new_start,
                        prod_start, (const int *)nullptr, parent, prank, stage, stage_off, next_id, cap, err);
 }
-template <typename R>
-void launch_fused_count(const DevConst<R> &k, const PView<R> &p, int isp, const StepClock *clk, int *cnt, int *pcnt,
-                        unsigned long long *mccr, int *cc, uint8_t *flag, R *stash, size_t stash_stride, int *err,
-                        hipStream_t s) {
-    const CountJob<R> J{k, p, isp, clk, cnt, pcnt, mccr, cc, flag, stash, stash_stride, err};
-    const int nb = count_blocks(k.Csize);
-    if (Recorder *r = launch_recorder()) {
-        r->add(isp == 0 ? &launch_m<CountJob<R>, k_fused_count_m<R, KIND_AR_ELECTRON>, 256>
-                        : &launch_m<CountJob<R>, k_fused_count_m<R, KIND_AR_ION>, 256>,
-               J, nb);
-        return;
-    }
-    if (isp == 0)
-        hipLaunchKernelGGL((k_fused_count<R, KIND_AR_ELECTRON>), dim3(nb), dim3(256), 0, s, J);
-    else
-        hipLaunchKernelGGL((k_fused_count<R, KIND_AR_ION>), dim3(nb), dim3(256), 0, s, J);
+// enqueues (or records) one launch of kernel K with job J, or of its merged-grid form KM
+template <typename J, void (*K)(J), void (*KM)(const J *, const uint32_t *)>
+static void launch_job(const J &job, int nb, hipStream_t s) {
+    if (Recorder *r = launch_recorder()) r->add(&launch_m<J, KM, 256>, job, nb);
+    else hipLaunchKernelGGL(K, dim3(nb), dim3(256), 0, s, job);
+}
+template <typename R, int CPW>
+static void launch_count_cpw(const CountJob<R> &e, const CountJob<R> &i, int which, hipStream_t s) {
+    const int nb = count_blocks(e.k.Csize, CPW);
+    if (which == 0) launch_job<CountJob<R>, k_fused_count<R, KIND_AR_ELECTRON, CPW>, k_fused_count_m<R, KIND_AR_ELECTRON, CPW>>(e, nb, s);
+    else if (which == 1) launch_job<CountJob<R>, k_fused_count<R, KIND_AR_ION, CPW>, k_fused_count_m<R, KIND_AR_ION, CPW>>(i, nb, s);
+    else launch_job<CountPair<R>, k_fused_count2<R, CPW>, k_fused_count2_m<R, CPW>>(CountPair<R>{e, i, nb}, 2 * nb, s);
 }
 template <typename R>
-void launch_fused_scatter(const DevConst<R> &k, const PView<R> &p, const PView<R> &q, const PView<R> &qion, int isp,
-                          const uint8_t *flag, const R *stash, size_t stash_stride, const int *base,
-                          const int *pbase_e, const int *pbase_i, const int *pid_off, const uint32_t *next_id,
-                          int cap, int cap_ion, int *err, hipStream_t s) {
-    const ScatterJob<R> J{k, p, q, qion, isp, flag, stash, stash_stride, base, pbase_e, pbase_i, pid_off, next_id,
-                          cap, cap_ion, err};
-    const int nb = cell_blocks(k.Csize);
-    if (Recorder *r = launch_recorder()) {
-        r->add(isp == 0 ? &launch_m<ScatterJob<R>, k_fused_scatter_m<R, KIND_AR_ELECTRON>, 256>
-                        : &launch_m<ScatterJob<R>, k_fused_scatter_m<R, KIND_AR_ION>, 256>,
-               J, nb);
-        return;
+void launch_fused_count(const DevConst<R> &k, const PView<R> &pe, const PView<R> &pi, int which, const StepClock *clk,
+                        int *cnt_e, int *cnt_i, int *pcnt, unsigned long long *mccr, int *cc, uint8_t *flag_e,
+                        uint8_t *flag_i, R *stash, size_t stash_stride, int *err, hipStream_t s) {
+    const CountJob<R> e{k, pe, 0, clk, cnt_e, pcnt, mccr, cc, flag_e, stash, stash_stride, err};
+    const CountJob<R> i{k, pi, 1, clk, cnt_i, nullptr, mccr, cc, flag_i, stash, stash_stride, err};
+    switch (count_cpw(k.Csize)) {
+    case 4: launch_count_cpw<R, 4>(e, i, which, s); break;
+    case 2: launch_count_cpw<R, 2>(e, i, which, s); break;
+    default: launch_count_cpw<R, 1>(e, i, which, s); break;
     }
-    if (isp == 0)
-        hipLaunchKernelGGL((k_fused_scatter<R, KIND_AR_ELECTRON>), dim3(nb), dim3(256), 0, s, J);
-    else
-        hipLaunchKernelGGL((k_fused_scatter<R, KIND_AR_ION>), dim3(nb), dim3(256), 0, s, J);
+}
+template <typename R>
+void launch_fused_scatter(const DevConst<R> &k, const PView<R> &pe, const PView<R> &pi, const PView<R> &qe,
+                          const PView<R> &qi, int which, const uint8_t *flag_e, const uint8_t *flag_i, const R *stash,
+                          size_t stash_stride, const int *base_e, const int *base_i, const int *pbase_e,
+                          const int *pbase_i, const int *pid_off, const uint32_t *next_id, int *err, hipStream_t s) {
+    const ScatterJob<R> e{k, pe, qe, qi, 0, flag_e, stash, stash_stride, base_e, pbase_e, pbase_i, pid_off, next_id,
+                          qe.cap, qi.cap, err};
+    const ScatterJob<R> i{k, pi, qi, qi, 1, flag_i, stash, stash_stride, base_i, pbase_i, pbase_i, pid_off, next_id,
+                          qi.cap, qi.cap, err};
+    const int nb = cell_blocks(k.Csize);
+    if (which == 0) launch_job<ScatterJob<R>, k_fused_scatter<R, KIND_AR_ELECTRON>, k_fused_scatter_m<R, KIND_AR_ELECTRON>>(e, nb, s);
+    else if (which == 1) launch_job<ScatterJob<R>, k_fused_scatter<R, KIND_AR_ION>, k_fused_scatter_m<R, KIND_AR_ION>>(i, nb, s);
+    else launch_job<ScatterPair<R>, k_fused_scatter2<R>, k_fused_scatter2_m<R>>(ScatterPair<R>{e, i, nb}, 2 * nb, s);
 }
 template <typename R>
 void launch_deposit(const DevConst<R> &k, const NodeConst<R> &n, const PView<R> *ps, R *part, R *den, R *sigma_sp,
@@ -1804,11 +1882,13 @@ void launch_scan(const int *in, int *out, int n, int *tmp, hipStream_t s) {
     template void launch_mcc_insert<R>(const DevConst<R> &, const PView<R> &, const PView<R> &, const int *,           \
                                        const int *, const PView<R> &, const int *, const R *, int, const uint32_t *,   \
                                        int, int *, hipStream_t);                                                       \
-    template void launch_fused_count<R>(const DevConst<R> &, const PView<R> &, int, const StepClock *, int *, int *,   \
-                                        unsigned long long *, int *, uint8_t *, R *, size_t, int *, hipStream_t);      \
+    template void launch_fused_count<R>(const DevConst<R> &, const PView<R> &, const PView<R> &, int,                  \
+                                        const StepClock *, int *, int *, int *, unsigned long long *, int *,          \
+                                        uint8_t *, uint8_t *, R *, size_t, int *, hipStream_t);                       \
     template void launch_fused_scatter<R>(const DevConst<R> &, const PView<R> &, const PView<R> &, const PView<R> &,   \
-                                          int, const uint8_t *, const R *, size_t, const int *, const int *,           \
-                                          const int *, const int *, const uint32_t *, int, int, int *, hipStream_t);   \
+                                          const PView<R> &, int, const uint8_t *, const uint8_t *, const R *, size_t,  \
+                                          const int *, const int *, const int *, const int *, const int *,             \
+                                          const uint32_t *, int *, hipStream_t);                                       \
     template void launch_deposit<R>(const DevConst<R> &, const NodeConst<R> &, const PView<R> *, R *, R *, R *, R *,   \
                                     R *, R *, const DepositExtras<R> *, hipStream_t);                                  \
     template void launch_eedf<R>(const PView<R> &, int, R, R, unsigned long long *, hipStream_t);               \

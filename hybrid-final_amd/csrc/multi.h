@@ -25,6 +25,26 @@ __device__ inline int multi_job(const uint32_t *map, int &lb) {
     return (int)(m >> MULTI_LB_BITS);
 }
 
+// A job record, read the way kernel arguments are: records never change while
+// a grid runs, so their loads go through the constant address space and stay
+// scalar.  As ordinary memory, which the kernel's own stores might change,
+// every pointer of a record was a vector load (the merged scatter held 121
+// VGPRs, the single-case one 54).
+template <typename J>
+__device__ inline const J &multi_record(const J *jobs, const uint32_t *map, int &lb) {
+    typedef const __attribute__((address_space(4))) J *Constant;
+    return *(const J *)(Constant)(uintptr_t)(jobs + multi_job(map, lb));   // by way of an integer: a plain cast folds away
+}
+
+// A pointer out of a record, known to the compiler as one to device memory (a
+// pointer loaded from memory could be one to LDS too, and its accesses would
+// be the slower flat ones).
+template <typename T>
+__device__ inline T *device_ptr(T *p) {
+    typedef __attribute__((address_space(1))) T *Global;
+    return (T *)(Global)(uintptr_t)p;
+}
+
 // launches a merged grid of `total` blocks over the job records at `jobs`
 typedef void (*MultiLaunchFn)(const void *jobs, const uint32_t *map, int total, hipStream_t s);
 
@@ -43,6 +63,7 @@ struct RecordedLaunch {
 
 struct Recorder {
     std::vector<RecordedLaunch> launches;
+    long long cells = 0;   // of all the cases that will share the launches (launch shapes follow the whole grid)
     template <typename J>
     void add(MultiLaunchFn fn, const J &job, int blocks) {
         RecordedLaunch r{fn, sizeof(J), alignof(J), blocks, {}};

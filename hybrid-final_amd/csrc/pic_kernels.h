@@ -153,15 +153,16 @@ void launch_mcc_insert(const DevConst<R> &, const PView<R> &, const PView<R> &, 
 // fused step: count pass (push, walls, MCC; collided particles written back
 // in place, flag byte per particle, ionisation products in stash, 6 arrays
 // of stash_stride) and scatter pass (sorted write of survivors and products)
+// which: 0 electrons, 1 ions, 2 both in one launch
 template <typename R>
-void launch_fused_count(const DevConst<R> &, const PView<R> &, int isp, const StepClock *clk, int *cnt, int *pcnt,
-                        unsigned long long *mccr, int *condcharge, uint8_t *flag, R *stash, size_t stash_stride,
-                        int *err, hipStream_t);
+void launch_fused_count(const DevConst<R> &, const PView<R> &pe, const PView<R> &pi, int which, const StepClock *clk,
+                        int *cnt_e, int *cnt_i, int *pcnt, unsigned long long *mccr, int *condcharge, uint8_t *flag_e,
+                        uint8_t *flag_i, R *stash, size_t stash_stride, int *err, hipStream_t);
 template <typename R>
-void launch_fused_scatter(const DevConst<R> &, const PView<R> &p, const PView<R> &q, const PView<R> &qion, int isp,
-                          const uint8_t *flag, const R *stash, size_t stash_stride, const int *base,
-                          const int *pbase_e, const int *pbase_i, const int *pid_off, const uint32_t *next_id, int cap,
-                          int cap_ion, int *err, hipStream_t);
+void launch_fused_scatter(const DevConst<R> &, const PView<R> &pe, const PView<R> &pi, const PView<R> &qe,
+                          const PView<R> &qi, int which, const uint8_t *flag_e, const uint8_t *flag_i, const R *stash,
+                          size_t stash_stride, const int *base_e, const int *base_i, const int *pbase_e,
+                          const int *pbase_i, const int *pid_off, const uint32_t *next_id, int *err, hipStream_t);
 template <typename R>
 void launch_deposit(const DevConst<R> &, const NodeConst<R> &, const PView<R> *, R *part, R *den, R *sigma_sp,
                     R *Sigma, R *Source, R *b, const DepositExtras<R> *ex, hipStream_t);

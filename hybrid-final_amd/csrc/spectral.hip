@@ -86,7 +86,7 @@ __global__ __launch_bounds__(RES_BLOCK) void k_residual64(ResidJob<RB> J) { resi
 template <typename RB>
 __global__ __launch_bounds__(RES_BLOCK) void k_residual64_m(const ResidJob<RB> *J, const uint32_t *map) {
     int lb;
-    const ResidJob<RB> &a = J[multi_job(map, lb)];
+    const ResidJob<RB> &a = multi_record(J, map, lb);
     residual64_body<RB>(a, lb);
 }
 
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void k_dgemm(GemmJob J) { dgemm_body<MODE>(J, 
 template <int MODE>
 __global__ __launch_bounds__(256) void k_dgemm_m(const GemmJob *J, const uint32_t *map) {
     int lb;
-    const GemmJob &a = J[multi_job(map, lb)];
+    const GemmJob &a = multi_record(J, map, lb);
     dgemm_body<MODE>(a, lb % a.gx, lb / a.gx);
 }
 
