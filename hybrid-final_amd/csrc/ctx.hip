@@ -172,7 +172,9 @@ struct Case : CaseBase {
     R *o2prob = nullptr, *o2fluid = nullptr, *o2bg = nullptr, *o2bg2 = nullptr, *o2bv2 = nullptr;
     R *o2stash[CHEM_MAXSP] = {nullptr};
     uint8_t *o2fate[CHEM_MAXSP] = {nullptr};
-    int *o2pcount = nullptr, *o2pstart = nullptr, *o2delreq = nullptr, *o2total = nullptr;
+    int *o2pcount = nullptr, *o2pstart = nullptr, *o2delreq = nullptr, *o2total = nullptr, *o2sums = nullptr;
+    O2Products *o2made = nullptr;   // nsp x G x ROUTE_SLOTS
+    uint8_t *o2any = nullptr;       // nsp x G
     unsigned long long *o2delcnt = nullptr;   // O- removed by electron detachment, per node, cumulative
     double *sum_den = nullptr, *sum_phi = nullptr, *sum_ex = nullptr, *sum_ey = nullptr;
     long long n_accum = 0;
@@ -218,7 +220,7 @@ struct Case : CaseBase {
                         inv_ent, pcol, pvalf, pmdf, pvald, pmdd, b64, x64, d_res, prank, pcnt, pid_off, total, alive,
                         ptotal, pstart, scan_tmp, cellp, next_id, mccr, condcharge, d_err, sum_den, sum_phi, sum_ex,
                         sum_ey, total2, alive2, clk, eedf, lost, sigma_hits, o2prob, o2fluid, o2bg, o2bg2, o2bv2,
-                        o2pcount, o2pstart, o2delreq, o2total, o2delcnt, diag_part, diag_hist, diag_cc_prev};
+                        o2pcount, o2pstart, o2delreq, o2total, o2sums, o2made, o2any, o2delcnt, diag_part, diag_hist, diag_cc_prev};
         for (void *p : ptrs)
             if (p) (void)hipFree(p);
         for (void *p : fl_bufs)
@@ -553,6 +555,9 @@ struct Case : CaseBase {
             HIPCHK(dalloc(&o2pcount, (size_t)nsp * G)); HIPCHK(dalloc(&o2pstart, (size_t)nsp * (G + 1)));
             HIPCHK(dalloc(&o2delreq, G));
             HIPCHK(dalloc(&o2total, (size_t)nsp * G));
+            HIPCHK(dalloc(&o2sums, o2_step_sums(G, nsp)));
+            HIPCHK(dalloc(&o2made, (size_t)nsp * G * ROUTE_SLOTS));
+            HIPCHK(dalloc(&o2any, (size_t)nsp * G));
             HIPCHK(dalloc(&o2delcnt, G));
             HIPCHK(hipMemsetAsync(o2delcnt, 0, (size_t)G * sizeof(unsigned long long), st));
             for (int s = 0; s < nsp; ++s) {
@@ -676,49 +681,14 @@ struct Case : CaseBase {
         HIPCHK(hipGetLastError());
         return 0;
     }
-    // Move and SortBounndary of a whole step: per species the push and the
-    // destination count in one pass, then the rest of the sort.  The same
-    // result as move() then sort_boundary() (no species' sort depends on
-    // another's push); the stage entry points keep the two passes apart.
-    // The bookkeeping between the two passes runs for all species at once:
-    // one totals launch, the scans three arrays per pass, one bases launch
-    // (the per-species totals live in o2total, which the collision step
-    // clears before its own use).
-    int move_sort() {
-        if (nsp > 5) return fail(-19, "staged whole steps take at most 5 species");
-        SortSpecies j{};
-        StagedSet<R> set{};
-        const int *in[CHEM_MAXSP];
-        int *out[CHEM_MAXSP];
-        for (int s = 0; s < nsp; ++s) {
-            set.p[s] = cur[s]; set.q[s] = nxt[s]; set.tag[s] = tag[s]; set.key[s] = key[s]; set.cnt[s] = cnt[s];
-            set.base[s] = base[s];
-            j.cnt[s] = cnt[s];
-            j.total[s] = o2total + (size_t)s * G;
-            j.start[s] = nxt[s].cell_start;
-            j.base[s] = base[s];
-            in[s] = j.total[s];
-            out[s] = nxt[s].cell_start;
-        }
-        launch_push_count<R>(kc, set, nsp, condcharge, st);
-        launch_totals_sp(G, nsp, inv_start, inv_ent, j, st);
-        for (int a = 0; a < nsp; a += 3) launch_scan_multi(std::min(3, nsp - a), in + a, out + a, G, scan_tmp, st);
-        launch_assign_bases_sp(G, nsp, inv_start, inv_ent, j, st);
-        launch_sort_scatter_all<R>(kc, set, nsp, d_err, st);
-        for (int s = 0; s < nsp; ++s) swap_species(s);
-        tag_valid = 0;
-        HIPCHK(hipGetLastError());
-        return 0;
-    }
     // oxygen chemistries: collide every species, remove the O- taken by
     // electron detachment, then rebuild every bucket with the products
     int mcc_o2() {
         const uint32_t step = (uint32_t)tstep;
         O2Set<R> set;
         for (int s = 0; s < nsp; ++s) { set.p[s] = cur[s]; set.fate[s] = o2fate[s]; set.stash[s] = o2stash[s]; }
-        launch_o2_probs<R>(oc, st);
+        launch_o2_probs<R>(oc, o2delreq, st);
         launch_fill_int(o2pcount, 0, nsp * G, st);
-        launch_fill_int(o2delreq, 0, G, st);
         launch_o2_collide<R>(oc, set, -1, step, mccr, o2pcount, o2delreq, st);   // all species
         launch_o2_victims<R>(oc, set, step, o2delreq, o2delcnt, st);
         O2Set<R> dst = set;
@@ -1317,16 +1287,35 @@ struct Case : CaseBase {
         HIPCHK(hipGetLastError());
         return 0;
     }
+    // the same for the oxygen chemistries' species (o2_step.hip)
+    int particle_stage_o2() {
+        O2Step<R> S2{};
+        for (int s = 0; s < nsp; ++s) {
+            S2.p[s] = cur[s]; S2.q[s] = nxt[s]; S2.tag[s] = tag[s]; S2.fate[s] = o2fate[s]; S2.stash[s] = o2stash[s];
+            S2.cnt[s] = cnt[s]; S2.base[s] = base[s];
+            S2.made[s] = o2made + (size_t)s * G * ROUTE_SLOTS;
+            S2.any[s] = o2any + (size_t)s * G;
+        }
+        S2.inv_start = inv_start; S2.inv_ent = inv_ent; S2.delreq = o2delreq; S2.delcnt = o2delcnt; S2.mccr = mccr;
+        S2.condcharge = condcharge; S2.err = d_err; S2.alive = o2total; S2.pstart = o2pstart; S2.sums = o2sums;
+        S2.clk = clk; S2.next_id = next_id;
+        launch_o2_step<R>(kc, oc, S2, st);
+        for (int s = 0; s < nsp; ++s) swap_species(s);
+        tag_valid = 0;
+        for (int m = 3; m < 7; ++m) mark(m);   // one stage to the timers
+        HIPCHK(hipGetLastError());
+        return 0;
+    }
     // one fused step enqueued on the stream (no host synchronisation); the
     // host buffer parity flips, the host clock does not move
     int enqueue_step() {
         if (int e = field_efield_fused()) return e;   // marks 1 between solve and E field
         mark(2);
-        if (int e = particle_stage_fused()) return e;
+        if (int e = gas ? particle_stage_o2() : particle_stage_fused()) return e;
         mark(7);
         // deposit + profile sums + id counter and clock advance in one node kernel
-        DepositExtras<R> ex{1, sum_den, sum_phi, sum_ex, sum_ey, tot, Ex, Ey, next_id, pstart + G, clk,
-                            (double)S.dt, spec_fin};
+        DepositExtras<R> ex{1, sum_den, sum_phi, sum_ex, sum_ey, tot, Ex, Ey, next_id, gas ? o2pstart + G : pstart + G,
+                            gas ? G + 1 : 0, clk, (double)S.dt, spec_fin};
         launch_deposit<R>(kc, nc, cur, part, den, sigma_sp, Sigma, Source, brhs, &ex, st);
         if (fluid_on) launch_fluid_step<R>(fl, den, mccr, P1, P2, st);
         HIPCHK(hipGetLastError());
@@ -1360,17 +1349,6 @@ struct Case : CaseBase {
         return 0;
     }
     int step_fused(int n) override {
-        if (gas == 1 || gas == 2) {
-            // the fused two-pass step is built for the argon chemistry; O2
-            // and Ar/O2 cases run the stages one by one
-            for (int i = 0; i < n; ++i) {
-                int e;
-                if ((e = advance_time()) || (e = field_solve()) || (e = efield()) || (e = move_sort()) ||
-                    (e = mcc()) || (e = deposit()) || (e = diagnostic()))
-                    return e;
-            }
-            return 0;
-        }
         if (int e = ensure_clock()) return e;
         // graphs need a fixed launch sequence: the separable field solve, no timers
         const bool graph = use_graph && spectral && !timing;

@@ -28,13 +28,6 @@ Recorder *&launch_recorder() {
 
 namespace {
 
-// a particle view with its pointers known as device memory
-template <typename R>
-__device__ inline PView<R> device_view(const PView<R> &p) {
-    return PView<R>{device_ptr(p.x), device_ptr(p.y), device_ptr(p.vx), device_ptr(p.vy), device_ptr(p.vz),
-                    device_ptr(p.id), device_ptr(p.cell_start), p.cap};
-}
-
 template <typename R>
 __device__ inline R wave_sum(R v) {
 #pragma unroll
@@ -86,25 +79,6 @@ __global__ __launch_bounds__(256) void k_push(DevConst<R> k, PView<R> p, int isp
     }
 }
 
-// side effects of a particle that leaves through a wall
-template <typename R>
-__device__ inline void wall_effects(const DevConst<R> &k, const Route &rt, int isp, int c, int code, R x, R y, R vx,
-                                    R vy, int *condcharge) {
-    if (rt.dest == -2) {
-        atomicAdd(&condcharge[isp * k.CondNUMR + rt.info], 1);
-    } else if (rt.dest == -1) {
-        atomicAdd(&k.lost[isp], 1);
-    } else if (rt.dest == -3) {
-        int mcid = code_mcid(code, k.ngy);
-        int sm = padded_index(c, mcid, k.ngy);
-        int pa, pb;
-        R a, b;
-        dielectric_split<R>(k.StructIdx, k.ngy, c, mcid, sm, x, y, vx, vy, pa, a, pb, b);
-        atomicAdd(&k.sigma_hits[(size_t)isp * k.Gsize + pa], sigma_fixed((double)a));
-        atomicAdd(&k.sigma_hits[(size_t)isp * k.Gsize + pb], sigma_fixed((double)b));
-    }
-}
-
 // ============================================================ staged: Sort count
 // key[k] = slot << 24 | rank within (cell, slot); -1 when the particle leaves
 template <typename R>
@@ -141,60 +115,6 @@ __global__ __launch_bounds__(256) void k_sort_count(DevConst<R> k, PView<R> p, i
 #pragma unroll
         for (int s = 0; s < ROUTE_SLOTS; ++s) cnt[c * ROUTE_SLOTS + s] = run[s];
     }
-}
-
-// ============================================================ staged: Move + Sort count
-// k_push and k_sort_count in one pass while the particle is in registers
-// (whole staged steps), every species in one launch (grid row = species):
-// the same positions, tags, keys, counts and wall side effects, one read of
-// the particle instead of two.
-template <typename R>
-__global__ __launch_bounds__(256) void k_push_count(DevConst<R> k, StagedSet<R> set, int *condcharge) {
-    int lane;
-    int c = wave_cell(k.ncy, k.ngy, k.Csize, lane);
-    if (c < 0) return;
-    const int isp = blockIdx.y;
-    const PView<R> p = set.p[isp];
-    uint8_t *tag = set.tag[isp];
-    int *key = set.key[isp], *cnt = set.cnt[isp];
-    int k0, k1;
-    cell_range(p, c, k0, k1);
-    const unsigned long long lt = lanes_below(lane);
-    int run = 0;   // lane s < ROUTE_SLOTS: survivors of slot s so far
-    if (k0 < k1) {
-        CellE<R> e;
-        e.load(k.Ex, k.Ey, c, k.ngy);
-        const R As = k.Ascale[isp];
-        for (int base = k0; base < k1; base += 64) {
-            const int kk = base + lane;
-            int slot = -1;
-            if (kk < k1) {
-                R x = p.x[kk], y = p.y[kk], vx = p.vx[kk], vy = p.vy[kk];
-                const int code = push_particle<R>(e.ews, e.ewn, e.ees, e.een, e.yws, e.ywn, e.yes, e.yen, As, k.dt_dx,
-                                                  k.dt_dy, x, y, vx, vy);
-                p.x[kk] = x; p.y[kk] = y; p.vx[kk] = vx; p.vy[kk] = vy;
-                tag[kk] = (uint8_t)code;
-                const Route rt = k.route[c * ROUTE_SLOTS + code];
-                if (rt.dest >= 0) slot = rt.info & 15;
-                else wall_effects<R>(k, rt, isp, c, code, x, y, vx, vy, condcharge);
-            }
-            // ranks over the slots present in these 64 (usually 2-4 of
-            // the 9): lane s holds slot s's running count
-            int rank = -1;
-            unsigned long long pend = __ballot(slot >= 0);
-            while (pend) {
-                const int first = __builtin_ctzll(pend);
-                const int sl = __builtin_amdgcn_readfirstlane(__shfl(slot, first, 64));
-                const unsigned long long m = __ballot(slot == sl);
-                const int before = __builtin_amdgcn_readlane(run, sl);
-                if (slot == sl) rank = before + __popcll(m & lt);
-                if (lane == sl) run += __popcll(m);
-                pend &= ~m;
-            }
-            if (kk < k1) key[kk] = slot < 0 ? -1 : ((slot << 24) | rank);
-        }
-    }
-    if (lane < ROUTE_SLOTS) cnt[c * ROUTE_SLOTS + lane] = run;
 }
 
 // ============================================================ bases
@@ -493,33 +413,6 @@ __global__ __launch_bounds__(BASES_TILE) void k_pair_scan_bases_m(const PairBase
 }
 
 
-// Totals and bases of the staged sort for every species in one launch each
-// (no products; grid row = species): the same per-destination sums and
-// entry bases as k_totals and k_assign_bases.
-__global__ void k_totals_sp(int Gsize, const int *inv_start, const int *inv_ent, SortSpecies j) {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = blockIdx.y;
-    if (d >= Gsize) return;
-    const int *cnt = j.cnt[s];
-    int a = 0;
-    for (int e = inv_start[d]; e < inv_start[d + 1]; ++e) a += cnt[inv_ent[e]];
-    j.total[s][d] = a;
-}
-
-__global__ void k_assign_bases_sp(int Gsize, const int *inv_start, const int *inv_ent, SortSpecies j) {
-    const int d = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = blockIdx.y;
-    if (d >= Gsize) return;
-    const int *cnt = j.cnt[s];
-    int *base = j.base[s];
-    int run = j.start[s][d];
-    for (int e = inv_start[d]; e < inv_start[d + 1]; ++e) {
-        const int ent = inv_ent[e];
-        base[ent] = run;
-        run += cnt[ent];
-    }
-}
-
 // ============================================================ staged: Sort scatter
 template <typename R>
 __global__ __launch_bounds__(256) void k_sort_scatter(DevConst<R> k, PView<R> p, PView<R> q, const uint8_t *tag,
@@ -527,33 +420,6 @@ __global__ __launch_bounds__(256) void k_sort_scatter(DevConst<R> k, PView<R> p,
     int lane;
     int c = wave_cell(k.ncy, k.ngy, k.Csize, lane);
     if (c < 0) return;
-    int k0, k1;
-    cell_range(p, c, k0, k1);
-    for (int kk = k0 + lane; kk < k1; kk += 64) {
-        int ky = key[kk];
-        if (ky < 0) continue;
-        int slot = ky >> 24, rank = ky & 0xffffff;
-        int code = tag[kk];
-        Route rt = k.route[c * ROUTE_SLOTS + code];
-        R x = p.x[kk], y = p.y[kk], vx = p.vx[kk], vy = p.vy[kk];
-        apply_reflect<R>(rt.info, x, y, vx, vy);
-        int pos = base[c * ROUTE_SLOTS + slot] + rank;
-        if (pos >= cap) { atomicOr(err, 1); continue; }
-        q.x[pos] = x; q.y[pos] = y; q.vx[pos] = vx; q.vy[pos] = vy; q.vz[pos] = p.vz[kk]; q.id[pos] = p.id[kk];
-    }
-}
-
-// k_sort_scatter for every species in one launch (grid row = species)
-template <typename R>
-__global__ __launch_bounds__(256) void k_sort_scatter_all(DevConst<R> k, StagedSet<R> set, int *err) {
-    int lane;
-    int c = wave_cell(k.ncy, k.ngy, k.Csize, lane);
-    if (c < 0) return;
-    const int isp = blockIdx.y;
-    const PView<R> p = set.p[isp], q = set.q[isp];
-    const uint8_t *tag = set.tag[isp];
-    const int *key = set.key[isp], *base = set.base[isp];
-    const int cap = q.cap;
     int k0, k1;
     cell_range(p, c, k0, k1);
     for (int kk = k0 + lane; kk < k1; kk += 64) {
@@ -683,14 +549,6 @@ struct FStage {
     R x[C], y[C], vx[C], vy[C], vz[C];
     uint32_t id[C];
 };
-
-// Orders the LDS accesses of one wavefront (the hardware already executes a
-// wave's LDS instructions in order; this keeps the compiler from moving
-// them) between a phase that writes slots and one that reads other lanes'.
-__device__ inline void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 // global -> LDS for particles [b0, b0+n), n >= 1.  Lanes past the end load the
 // last particle again (same cache line, never read back), so the 6*C/64
@@ -1268,8 +1126,7 @@ __device__ __forceinline__ void deposit_nodes_body(const DepNodesJob<R> &J, int 
         if (g == 0) spec_decide(rr, bb, ex.fin.tol, 1, ex.fin.s, ex.fin.res);
     }
     if (ex.on && g == 0) {
-        const uint32_t add = (uint32_t)*ex.prod_total_end;
-        for (int s = 0; s < n.nsp; ++s) ex.next_id[s] += add;
+        for (int s = 0; s < n.nsp; ++s) ex.next_id[s] += (uint32_t)ex.prod_total_end[s * ex.prod_stride];
         // the next step: same arithmetic as the host's t = tstep * dt
         const uint32_t nstep = ex.clk->step + 1u;
         ex.clk->step = nstep;
@@ -1682,14 +1539,6 @@ void launch_sort_count(const DevConst<R> &k, const PView<R> &p, int isp, const u
     hipLaunchKernelGGL(k_sort_count<R>, dim3(cell_blocks(k.Csize)), dim3(256), 0, s, k, p, isp, tag, key, cnt, cc);
 }
 template <typename R>
-void launch_push_count(const DevConst<R> &k, const StagedSet<R> &set, int nsp, int *cc, hipStream_t s) {
-    hipLaunchKernelGGL(k_push_count<R>, dim3(cell_blocks(k.Csize), nsp), dim3(256), 0, s, k, set, cc);
-}
-template <typename R>
-void launch_sort_scatter_all(const DevConst<R> &k, const StagedSet<R> &set, int nsp, int *err, hipStream_t s) {
-    hipLaunchKernelGGL(k_sort_scatter_all<R>, dim3(cell_blocks(k.Csize), nsp), dim3(256), 0, s, k, set, err);
-}
-template <typename R>
 void launch_sort_scatter(const DevConst<R> &k, const PView<R> &p, const PView<R> &q, const uint8_t *tag,
                          const int *key, const int *base, int cap, int *err, hipStream_t s) {
     hipLaunchKernelGGL(k_sort_scatter<R>, dim3(cell_blocks(k.Csize)), dim3(256), 0, s, k, p, q, tag, key, base, cap, err);
@@ -1849,15 +1698,6 @@ void launch_bases_pair(int G, const int *inv_start, const int *inv_ent, const in
 int scan_tmp_ints(int n) { return 3 * ((n + BASES_TILE - 1) / BASES_TILE) + 3; }
 // exclusive scans of k <= 3 arrays of n ints: out[a][0..n], out[a][n] = total;
 // tmp holds scan_tmp_ints(n) ints
-void launch_totals_sp(int Gsize, int nsp, const int *inv_start, const int *inv_ent, const SortSpecies &j,
-                      hipStream_t s) {
-    hipLaunchKernelGGL(k_totals_sp, dim3(node_blocks(Gsize), nsp), dim3(256), 0, s, Gsize, inv_start, inv_ent, j);
-}
-void launch_assign_bases_sp(int Gsize, int nsp, const int *inv_start, const int *inv_ent, const SortSpecies &j,
-                            hipStream_t s) {
-    hipLaunchKernelGGL(k_assign_bases_sp, dim3(node_blocks(Gsize), nsp), dim3(256), 0, s, Gsize, inv_start, inv_ent,
-                       j);
-}
 void launch_scan_multi(int k, const int *const *in, int *const *out, int n, int *tmp, hipStream_t s) {
     const int nt = std::max(1, (n + SCAN_TILE - 1) / SCAN_TILE);
     ScanJobs J{};
@@ -1871,8 +1711,6 @@ void launch_scan(const int *in, int *out, int n, int *tmp, hipStream_t s) {
 
 #define INST(R)                                                                                                         \
     template void launch_push<R>(const DevConst<R> &, const PView<R> &, int, uint8_t *, hipStream_t);                 \
-    template void launch_push_count<R>(const DevConst<R> &, const StagedSet<R> &, int, int *, hipStream_t);          \
-    template void launch_sort_scatter_all<R>(const DevConst<R> &, const StagedSet<R> &, int, int *, hipStream_t);    \
     template void launch_sort_count<R>(const DevConst<R> &, const PView<R> &, int, const uint8_t *, int *, int *,      \
                                        int *, hipStream_t);                                                            \
     template void launch_sort_scatter<R>(const DevConst<R> &, const PView<R> &, const PView<R> &, const uint8_t *,     \

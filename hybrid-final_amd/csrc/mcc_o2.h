@@ -52,7 +52,8 @@ struct O2Set {
     R *stash[CHEM_MAXSP];     // 6 arrays of p[s].cap: product 0 velocity, product 1 velocity
 };
 
-template <typename R> void launch_o2_probs(const O2Const<R> &k, hipStream_t s);
+// target probabilities per node; clears delreq too when it is given
+template <typename R> void launch_o2_probs(const O2Const<R> &k, int *delreq, hipStream_t s);
 // collisions of species isp (every species when isp < 0), in place;
 // counts products per (species, node) into pcount (nsp x G), O- removal
 // requests per node into delreq, and the O- actually removed for them per
@@ -75,6 +76,35 @@ void launch_o2_totals(const O2Const<R> &k, const O2Set<R> &set, const int *pcoun
 template <typename R>
 void launch_o2_scatter_all(const O2Const<R> &k, const O2Set<R> &set, const O2Set<R> &dst, const int *pstart,
                            const uint32_t *next_id, int *err, hipStream_t s);
+// ---- whole steps in two passes (o2_step.hip)
+struct O2Products {
+    unsigned long long lo, hi;   // counts per product species, 21 bits each: 0-2, 3-4
+};
+template <typename R>
+struct O2Step {
+    PView<R> p[CHEM_MAXSP], q[CHEM_MAXSP];   // buckets before and after the step
+    uint8_t *tag[CHEM_MAXSP];                // per particle: O2T_* flags of the first pass
+    uint8_t *fate[CHEM_MAXSP];               // product species of particles with O2T_PROD (O2F_* layout)
+    R *stash[CHEM_MAXSP];                    // product velocities, as in O2Set
+    int *cnt[CHEM_MAXSP], *base[CHEM_MAXSP]; // per (cell, slot): survivors, and where they start
+    O2Products *made[CHEM_MAXSP];            // per (cell, slot): products; then those placed before them
+    uint8_t *any[CHEM_MAXSP];                // per cell: it has products (made is only kept then)
+    const int *inv_start, *inv_ent;
+    int *delreq;
+    unsigned long long *delcnt, *mccr;
+    int *condcharge, *err;
+    int *alive;                              // nsp x G: where a destination's products start
+    int *pstart;                             // nsp x (G + 1): product order
+    int *sums;                               // 2 nsp x tiles of 256 nodes
+    const StepClock *clk;
+    const uint32_t *next_id;
+};
+// pushes every particle, applies walls and collisions, and writes the sorted
+// buckets q; the same result as the stages one by one
+template <typename R>
+void launch_o2_step(const DevConst<R> &k, const O2Const<R> &oc, const O2Step<R> &st, hipStream_t s);
+int o2_step_sums(int G, int nsp);   // ints of O2Step::sums
+
 // next_id[t] += product total of species t (pstart is nsp x (G+1))
 void launch_o2_bump_ids(uint32_t *next_id, const int *pstart, int G, int nsp, hipStream_t s);
 

@@ -27,54 +27,27 @@
 // (handlers and target tests).
 #include <hip/hip_runtime.h>
 
-#include "mcc_o2.h"
+#include "mcc_o2_device.h"
 
 namespace pic {
 
 namespace {
 
-struct ChemRow {
-    int r, sum, type, emode;
-    double gain;
-    int p0, p1, th;
-};
-struct ChemGroup {
-    int sp, flag, sig, first, n, vsrc;
-};
-struct ChemTarget {
-    int sp, flag, sig, kind, idx;
-};
-
-// both chemistries in one form: O2 rows subtract their own threshold, and
-// its O2+ and O+ collide in the frame of a neutral at BackVel1
-#define PIC_O2_ROW(r, sm, ty, em, g, a, b) {r, sm, ty, em, g, a, b, r},
-#define PIC_ARO2_ROW(r, sm, ty, em, g, a, b, th) {r, sm, ty, em, g, a, b, th},
-#define PIC_O2_GRP(s, f, sg, fi, n) {s, f, sg, fi, n, (s) == 1 || (s) == 2 ? 1 : 0},
-#define PIC_ARO2_GRP(s, f, sg, fi, n, v) {s, f, sg, fi, n, v},
-#define PIC_TGT(s, f, sg, kd, ix) {s, f, sg, kd, ix},
-__constant__ ChemRow kRow[2][CHEM_MAXROWS] = {{O2_REACTIONS(PIC_O2_ROW)}, {ARO2_REACTIONS(PIC_ARO2_ROW)}};
-__constant__ ChemGroup kGrp[2][CHEM_MAXGROUPS] = {{O2_GROUPS(PIC_O2_GRP)}, {ARO2_GROUPS(PIC_ARO2_GRP)}};
-__constant__ ChemTarget kTgt[2][CHEM_MAXTARGETS] = {{O2_TARGETS(PIC_TGT)}, {ARO2_TARGETS(PIC_TGT)}};
-__constant__ int kGroup0[2][CHEM_MAXSP] = {O2_GROUP0, ARO2_GROUP0};
-__constant__ int kNGroup[2][CHEM_MAXSP] = {O2_NGROUP, ARO2_NGROUP};
-#undef PIC_O2_ROW
-#undef PIC_ARO2_ROW
-#undef PIC_O2_GRP
-#undef PIC_ARO2_GRP
-#undef PIC_TGT
-
 // Target probabilities: P_j = P_{j-1} + 1 - exp(-dt_s sigv n), summed in
 // that order as the reference writes it (src/cuda_mccO2.cu:880-930,
-// src/cuda_mccArO2.cu:1144-1205).
+// src/cuda_mccArO2.cu:1144-1205).  One thread per node and species: a species'
+// sum is a serial chain of exponentials (all species in one thread took
+// 18.9 us at 257x129 nodes).  delreq, when given, is cleared on the way.
 template <typename R>
-__global__ __launch_bounds__(256) void k_o2_probs(O2Const<R> k) {
+__global__ __launch_bounds__(256) void k_o2_probs(O2Const<R> k, int *delreq) {
     const int g = blockIdx.x * 256 + threadIdx.x;
+    const int sp = blockIdx.y;
     if (g >= k.G) return;
+    if (delreq && sp == 0) delreq[g] = 0;
     R acc = 0;
-    int sp = -1;
-    for (int t = 0; t < k.ntgt; ++t) {
+    const int t0 = kGroup0[k.chem][sp], t1 = t0 + kNGroup[k.chem][sp];
+    for (int t = t0; t < t1; ++t) {
         const ChemTarget T = kTgt[k.chem][t];
-        if (T.sp != sp) { sp = T.sp; acc = 0; }
         R x = (((k.sub_mask >> T.sp) & 1) ? k.dtm : k.dt) * k.sigv[T.sig];
         if (T.kind == 0) x = x * (T.idx ? k.BackDen2[g] : k.BackDen1[g]);
         else if (T.kind == 1) x = x * k.FluidN[(size_t)T.idx * k.G + g];
@@ -82,128 +55,6 @@ __global__ __launch_bounds__(256) void k_o2_probs(O2Const<R> k) {
         acc = (acc + (R)1) - (R)dm_exp(-(double)x);
         k.prob[(size_t)g * k.ntgt + t] = acc;
     }
-}
-
-template <typename R>
-__device__ inline void o2_maxwell(const O2Const<R> &k, R vti, Stream &st, R &vx, R &vy, R &vz) {
-    const int n = (int)((R)(k.nvel - 1) * st.u<R>());
-    const R rphi = st.u<R>(), rthe = st.u<R>();
-    maxwell_draw<R>(vx, vy, vz, k.vsave[n], vti, rphi, rthe);
-}
-
-// One collision of a particle of species isp with the target of group grp.
-// Returns the reaction (or -1 for a null collision); vx..vz are updated for
-// a survivor, and dead / products / detach describe the rest.
-template <typename R>
-__device__ inline int o2_handle(const O2Const<R> &k, int isp, int grp, int c, Stream &st, R &vx, R &vy, R &vz,
-                                int &dead, int ps[2], R pv[2][3], int &np, int &detach) {
-    const ChemGroup g = kGrp[k.chem][grp];
-    R vnx = 0, vny = 0, vnz = 0;
-    const bool heavy = g.vsrc != 0;   // positive ions collide in the neutral's frame
-    if (heavy) o2_maxwell<R>(k, g.vsrc == 2 ? k.BackVel2[c] : k.BackVel1[c], st, vnx, vny, vnz);
-    R VX = vx - vnx, VY = vy - vny, VZ = vz - vnz;
-    const R dum = VX * VX + VY * VY + VZ * VZ;
-    R vel = rsqrt_ieee<R>(dum);
-    if (!heavy) { VX /= vel; VY /= vel; VZ /= vel; }
-    R engy = k.Escale[isp] * dum;
-    const R R1 = st.u<R>() * k.sigv[g.sig] / vel;
-    ArXs<R> xs;
-    xs.init(k, engy);
-    R sum = 0;
-    int hit = -1;
-    for (int q = g.first; q < g.first + g.n; ++q) {
-        const int r = kRow[k.chem][q].r;
-        if (engy > k.Th_e[r]) {
-            const R sg = xs.sigma(k, r);
-            sum = kRow[k.chem][q].sum ? sum + sg : sg;
-            if (R1 <= sum) { hit = q; break; }
-        }
-    }
-    if (hit < 0) return -1;
-    const ChemRow row = kRow[k.chem][hit];
-    const R Es = k.Escale[isp];
-    switch (row.type) {
-    case O2T_LOSS:
-    case O2T_ION:
-    case O2T_DETACH: {
-        if (row.emode == O2E_LOSS) {
-            engy -= k.Th_e[row.th];
-            vel = rsqrt_ieee<R>(rabs<R>(engy) / Es);
-        } else if (row.emode == O2E_GAIN) {
-            engy += (R)row.gain;
-            vel = rsqrt_ieee<R>(rabs<R>(engy) / Es);
-        }
-        if (row.type == O2T_ION) {
-            for (int slot = 0; slot < 2; ++slot) {
-                const int sp = slot ? row.p1 : row.p0;
-                ps[np] = sp;
-                if (sp == 0) { pv[np][0] = VX; pv[np][1] = VY; pv[np][2] = VZ; }
-                else o2_maxwell<R>(k, k.BackVel1[c], st, pv[np][0], pv[np][1], pv[np][2]);
-                ++np;
-            }
-        } else if (row.type == O2T_DETACH) {
-            ps[np] = 0; pv[np][0] = VX; pv[np][1] = VY; pv[np][2] = VZ; ++np;
-            detach = 1;
-        }
-        const R a = st.u<R>(), b = st.u<R>();
-        anewvel<R>(engy, vel, VX, VY, VZ, a, b);
-        vx = VX; vy = VY; vz = VZ;
-        break;
-    }
-    case O2T_IONSHARE: {
-        engy -= k.Th_e[row.th];
-        const R u = st.u<R>();
-        const R rengy = (R)10 * PMath<R>::tan(u * PMath<R>::atan(engy / (R)20));
-        engy -= rengy;
-        const R velr = rsqrt_ieee<R>(rabs<R>(rengy) / Es);
-        const R vel2 = rsqrt_ieee<R>(rabs<R>(engy) / Es);
-        for (int slot = 0; slot < 2; ++slot) {
-            const int sp = slot ? row.p1 : row.p0;
-            ps[np] = sp;
-            if (sp == 0) {
-                R ex = VX, ey = VY, ez = VZ;
-                const R a = st.u<R>(), b = st.u<R>();
-                anewvel<R>(rengy, velr, ex, ey, ez, a, b);
-                pv[np][0] = ex; pv[np][1] = ey; pv[np][2] = ez;
-            } else {
-                o2_maxwell<R>(k, k.BackVel1[c], st, pv[np][0], pv[np][1], pv[np][2]);
-            }
-            ++np;
-        }
-        const R a = st.u<R>(), b = st.u<R>();
-        anewvel<R>(engy, vel2, VX, VY, VZ, a, b);
-        vx = VX; vy = VY; vz = VZ;
-        break;
-    }
-    case O2T_ATTACH:
-        dead = 1;
-        ps[np] = row.p0;
-        o2_maxwell<R>(k, k.BackVel1[c], st, pv[np][0], pv[np][1], pv[np][2]);
-        ++np;
-        break;
-    case O2T_DEL:
-        dead = 1;
-        break;
-    case O2T_SCAT: {
-        const R a = st.u<R>(), b = st.u<R>();
-        newvel_ionsc<R>(VX, VY, VZ, vel, a, b);
-        if (heavy) { vx = VX + vnx; vy = VY + vny; vz = VZ + vnz; }
-        else { vx = VX; vy = VY; vz = VZ; }
-        break;
-    }
-    case O2T_CXKEEP:
-        vx = vnx; vy = vny; vz = vnz;
-        break;
-    case O2T_CXTO:
-        dead = 1;
-        ps[np] = row.p0; pv[np][0] = vnx; pv[np][1] = vny; pv[np][2] = vnz; ++np;
-        break;
-    default:   // O2T_NEGDET
-        dead = 1;
-        ps[np] = 0; pv[np][0] = VX; pv[np][1] = VY; pv[np][2] = VZ; ++np;
-        break;
-    }
-    return row.r;
 }
 
 constexpr int O2_WAVES = 4;     // waves per block, one cell each
@@ -229,6 +80,9 @@ __global__ __launch_bounds__(256) void k_o2_collide(O2Const<R> k, O2Set<R> set, 
     __shared__ unsigned char q_c[O2_WAVES][O2_QCAP];
     __shared__ int c_r[O2_WAVES][O2_CPW][CHEM_MAXROWS + 1];   // events per (cell, row); last = detachments
     __shared__ int c_p[O2_WAVES][O2_CPW][CHEM_MAXSP];         // products per (cell, species)
+    __shared__ SearchRow<R> tab[CHEM_MAXROWS];
+    load_search(k, tab);
+    __syncthreads();
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (isp < 0) isp = blockIdx.y;
     const int w0 = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6)) * O2_CPW;
@@ -288,12 +142,11 @@ __global__ __launch_bounds__(256) void k_o2_collide(O2Const<R> k, O2Set<R> set, 
         st.init(k.seed, p.id[kk], step, tag);
         st.seek(jc);
         const R R1 = st.u<R>();
-        int flag = 0;
-        while (flag < ng - 1 && R1 > P[flag]) ++flag;
+        const int flag = o2_target(P, ng, R1);
         R vx = p.vx[kk], vy = p.vy[kk], vz = p.vz[kk];
         int dead = 0, np = 0, detach = 0, ps[2] = {-1, -1};
         R pv[2][3];
-        const int r = o2_handle<R>(k, isp, g0 + flag, c, st, vx, vy, vz, dead, ps, pv, np, detach);
+        const int r = o2_handle<R>(k, tab, isp, g0 + flag, c, st, vx, vy, vz, dead, ps, pv, np, detach);
         uint8_t f = 0;
         if (r >= 0) {
             atomicAdd(&c_r[wv][kq][r], 1);
@@ -623,8 +476,8 @@ inline int wave_blocks(int Csize) { return (Csize + O2_WAVES - 1) / O2_WAVES; }
 }  // namespace
 
 template <typename R>
-void launch_o2_probs(const O2Const<R> &k, hipStream_t s) {
-    hipLaunchKernelGGL(k_o2_probs<R>, dim3((k.G + 255) / 256), dim3(256), 0, s, k);
+void launch_o2_probs(const O2Const<R> &k, int *delreq, hipStream_t s) {
+    hipLaunchKernelGGL(k_o2_probs<R>, dim3((k.G + 255) / 256, k.nsp), dim3(256), 0, s, k, delreq);
 }
 template <typename R>
 void launch_o2_collide(const O2Const<R> &k, const O2Set<R> &set, int isp, uint32_t step, unsigned long long *mccr,
@@ -656,7 +509,7 @@ void launch_o2_bump_ids(uint32_t *next_id, const int *pstart, int G, int nsp, hi
 }
 
 #define INST(R)                                                                                                       \
-    template void launch_o2_probs<R>(const O2Const<R> &, hipStream_t);                                               \
+    template void launch_o2_probs<R>(const O2Const<R> &, int *, hipStream_t);                                        \
     template void launch_o2_collide<R>(const O2Const<R> &, const O2Set<R> &, int, uint32_t, unsigned long long *,     \
                                        int *, int *, hipStream_t);                                                   \
     template void launch_o2_victims<R>(const O2Const<R> &, const O2Set<R> &, uint32_t, const int *,                  \

@@ -103,14 +103,15 @@ struct Exchange {
         if ((uint32_t)(v >> 32) != want) {
             const u64 t0 = __builtin_amdgcn_s_memrealtime();
             for (int n = 1;; ++n) {
-                v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if ((uint32_t)(v >> 32) == want) break;
-                if (__builtin_amdgcn_s_memrealtime() - t0 > spin_limit) {
+                // the limit first: with a limit of zero no word may be waited for
+                if (__builtin_amdgcn_s_memrealtime() - t0 >= spin_limit) {
                     __hip_atomic_store(&st->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     return false;
                 }
                 if ((n & 63) == 0 && __hip_atomic_load(&st->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
                     return false;
+                v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((uint32_t)(v >> 32) == want) break;
             }
         }
         data = (uint32_t)v;

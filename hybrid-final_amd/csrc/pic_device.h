@@ -244,6 +244,25 @@ __host__ __device__ inline int padded_index(int ID, int MCID, int ngy) {
     return (ID + ngy + 2 + x) + MCID;
 }
 
+// side effects of a particle that leaves through a wall
+template <typename R>
+__device__ inline void wall_effects(const DevConst<R> &k, const Route &rt, int isp, int c, int code, R x, R y, R vx,
+                                    R vy, int *condcharge) {
+    if (rt.dest == -2) {
+        atomicAdd(&condcharge[isp * k.CondNUMR + rt.info], 1);
+    } else if (rt.dest == -1) {
+        atomicAdd(&k.lost[isp], 1);
+    } else if (rt.dest == -3) {
+        int mcid = code_mcid(code, k.ngy);
+        int sm = padded_index(c, mcid, k.ngy);
+        int pa, pb;
+        R a, b;
+        dielectric_split<R>(k.StructIdx, k.ngy, c, mcid, sm, x, y, vx, vy, pa, a, pb, b);
+        atomicAdd(&k.sigma_hits[(size_t)isp * k.Gsize + pa], sigma_fixed((double)a));
+        atomicAdd(&k.sigma_hits[(size_t)isp * k.Gsize + pb], sigma_fixed((double)b));
+    }
+}
+
 // ---------------------------------------------------------------- elementary functions
 // In the path's precision: the FP32 path uses the single-precision
 // deterministic routines of detmath.h, the FP64 path the double ones.
@@ -272,33 +291,39 @@ template <> struct PMath<double> {
 // scratch.
 template <typename R>
 struct ArXs {
-    int mode;       // 0 zero energy, 1 below the table, 2 above it, 3 last row, 4 inside
-    int ee2;
+    int mode;         // 0 zero energy, 1 below the table, 2 above it, 3 last row, 4 inside
+    int row1, row2;   // table rows of this energy (the same one twice outside the inside)
     R a1, a2;
-    double tail;    // dm_exp(-(lengy - xe[N-1])) above the table
+    double tail;      // dm_exp(-(lengy - xe[N-1])) above the table
     template <class K>
     __device__ void init(const K &k, R engy) {
         const int N = k.nlogx;
-        if (engy == 0) { mode = 0; return; }
+        mode = row1 = row2 = 0;
+        a1 = a2 = 0;
+        tail = 0;
+        if (engy == 0) return;
         const R lengy = PMath<R>::log10(engy);
         const R ee1 = k.idLOGX * (lengy - k.xe[0]);
-        ee2 = (int)ee1;
+        const int ee2 = (int)ee1;
         a1 = ee1 - (R)ee2;
         a2 = 1 - a1;
         if (lengy < k.xe[0]) mode = 1;
-        else if (lengy > k.xe[N - 1]) { mode = 2; tail = dm_exp(-(double)(lengy - k.xe[N - 1])); }
-        else if (ee2 >= N - 1) mode = 3;
-        else mode = 4;
+        else if (lengy > k.xe[N - 1]) { mode = 2; row1 = row2 = N - 1; tail = dm_exp(-(double)(lengy - k.xe[N - 1])); }
+        else if (ee2 >= N - 1) { mode = 3; row1 = row2 = N - 1; }
+        else { mode = 4; row1 = ee2; row2 = ee2 + 1; }
     }
+    // the two table values are loaded whatever the mode, so the lookups of
+    // several reactions can be in flight together
     template <class K>
     __device__ R sigma(const K &k, int r) const {
-        const int N = k.nlogx, T = k.TnRct;
+        const int T = k.TnRct;
+        const R c1 = k.cx[row1 * T + r], c2 = k.cx[row2 * T + r];
         switch (mode) {
         case 0: return 0;
-        case 1: return k.cx[r];
-        case 2: return (R)((double)k.cx[(N - 1) * T + r] * 0.1 * tail);
-        case 3: return k.cx[(N - 1) * T + r];
-        default: return a2 * k.cx[ee2 * T + r] + a1 * k.cx[(ee2 + 1) * T + r];
+        case 1:
+        case 3: return c1;
+        case 2: return (R)((double)c1 * 0.1 * tail);
+        default: return a2 * c1 + a1 * c2;
         }
     }
 };
@@ -399,11 +424,12 @@ __device__ inline int mcc_ar_ion_collide(const DevConst<R> &k, int node, Stream 
     ArXs<R> xs;
     xs.init(k, engy);
     R sum = xs.sigma(k, 5);
+    const R s6 = xs.sigma(k, 6);
     if (R1 <= sum) {
         vx = vnx; vy = vny; vz = vnz;
         return 5;
     }
-    if (R1 <= (sum += xs.sigma(k, 6))) {
+    if (R1 <= (sum += s6)) {
         R a = st.u<R>(), b = st.u<R>();
         newvel_ionsc<R>(VX, VY, VZ, vel, a, b);
         vx = VX + vnx; vy = VY + vny; vz = VZ + vnz;
@@ -457,15 +483,17 @@ __device__ inline int mcc_ar_electron_collide(const DevConst<R> &k, int node, R 
     const R Es = k.Escale[0];
     ArXs<R> xs;
     xs.init(k, engy);   // every comparison below uses this energy
+    // all lookups at once: one after the other, each waits for its own load
+    const R s04 = xs.sigma(k, target == 0 ? 0 : 4), s1 = xs.sigma(k, 1), s2 = xs.sigma(k, 2), s3 = xs.sigma(k, 3);
     if (target == 0) {
         R2 = st.u<R>() * k.sigv[0] / vel;
-        sum = xs.sigma(k, 0);
+        sum = s04;
         if (R2 <= sum) { type = 0; ev = 0; }
-        else if (engy > k.Th_e[1] && R2 <= (sum += xs.sigma(k, 1))) {
+        else if (engy > k.Th_e[1] && R2 <= (sum += s1)) {
             type = 0; ev = 1; engy -= k.Th_e[1]; vel = rsqrt_ieee<R>(rabs<R>(engy) / Es);
-        } else if (engy > k.Th_e[2] && R2 <= (sum += xs.sigma(k, 2))) {
+        } else if (engy > k.Th_e[2] && R2 <= (sum += s2)) {
             type = 0; ev = 2; engy -= k.Th_e[2]; vel = rsqrt_ieee<R>(rabs<R>(engy) / Es);
-        } else if (engy > k.Th_e[3] && R2 <= (sum += xs.sigma(k, 3))) {
+        } else if (engy > k.Th_e[3] && R2 <= (sum += s3)) {
             type = 2; ev = 3; engy -= k.Th_e[3];
             R u = st.u<R>();
             rengy = (R)10 * PMath<R>::tan(u * PMath<R>::atan(engy / (R)20));
@@ -475,7 +503,7 @@ __device__ inline int mcc_ar_electron_collide(const DevConst<R> &k, int node, R 
         }
     } else {
         R2 = st.u<R>() * k.sigv[1] / vel;
-        sum = xs.sigma(k, 4);
+        sum = s04;
         if (engy > k.Th_e[4] && R2 <= sum) {
             type = 2; ev = 4; engy -= k.Th_e[4];
             R u = st.u<R>();

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "multi.h"
 #include "pic_device.h"
 
 namespace pic {
@@ -51,6 +52,21 @@ __device__ inline void cell_range(const PView<R> &p, int c, int &k0, int &k1) {
 
 __device__ inline unsigned long long lanes_below(int lane) {
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));
+}
+
+// Orders the LDS accesses of one wavefront (the hardware already executes a
+// wave's LDS instructions in order; this keeps the compiler from moving
+// them) between a phase that writes slots and one that reads other lanes'.
+__device__ inline void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// a particle view with its pointers known as device memory
+template <typename R>
+__device__ inline PView<R> device_view(const PView<R> &p) {
+    return PView<R>{device_ptr(p.x), device_ptr(p.y), device_ptr(p.vx), device_ptr(p.vy), device_ptr(p.vz),
+                    device_ptr(p.id), device_ptr(p.cell_start), p.cap};
 }
 
 // particle views of all species of a case (kernel argument)
@@ -111,7 +127,8 @@ struct DepositExtras {
     double *sden, *sphi, *sex, *sey;
     const R *tot, *Ex, *Ey;
     uint32_t *next_id;
-    const int *prod_total_end;
+    const int *prod_total_end;   // products of the step, per species at this stride (0: one count for all)
+    int prod_stride;
     StepClock *clk;
     double dt;
     SpecFinal fin;   // the field solve's last convergence test
@@ -126,19 +143,6 @@ struct VoltConst {
 };
 
 template <typename R> void launch_push(const DevConst<R> &, const PView<R> &, int, uint8_t *, hipStream_t);
-// every species of a staged step, for the all-species launches of a whole
-// step (push + count, sort scatter)
-template <typename R>
-struct StagedSet {
-    PView<R> p[5], q[5];
-    uint8_t *tag[5];
-    int *key[5], *cnt[5];
-    const int *base[5];
-};
-template <typename R>
-void launch_push_count(const DevConst<R> &, const StagedSet<R> &, int nsp, int *condcharge, hipStream_t);
-template <typename R>
-void launch_sort_scatter_all(const DevConst<R> &, const StagedSet<R> &, int nsp, int *err, hipStream_t);
 template <typename R>
 void launch_sort_count(const DevConst<R> &, const PView<R> &, int, const uint8_t *, int *, int *, int *, hipStream_t);
 template <typename R>
@@ -189,18 +193,6 @@ void launch_assign_bases(int, const int *, const int *, const int *, const int *
 void launch_scan(const int *in, int *out, int n, int *tmp, hipStream_t s);
 int scan_tmp_ints(int n);
 void launch_scan_multi(int k, const int *const *in, int *const *out, int n, int *tmp, hipStream_t s);
-// the staged sort's per-species arrays, for its all-species launches
-constexpr int SORT_MAXSP = 8;
-struct SortSpecies {
-    const int *cnt[SORT_MAXSP];
-    int *total[SORT_MAXSP];
-    const int *start[SORT_MAXSP];
-    int *base[SORT_MAXSP];
-};
-void launch_totals_sp(int Gsize, int nsp, const int *inv_start, const int *inv_ent, const SortSpecies &j,
-                      hipStream_t s);
-void launch_assign_bases_sp(int Gsize, int nsp, const int *inv_start, const int *inv_ent, const SortSpecies &j,
-                            hipStream_t s);
 // fused step, between the passes: per-destination totals of both species,
 // their scans (cell_start of both species, product order) and the base of
 // every (source cell, slot) entry; tmp holds scan_tmp_ints(G) ints

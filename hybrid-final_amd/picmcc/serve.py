@@ -52,6 +52,7 @@ def footprint_estimate(deck, precision=FP32_REFINED):
     per_slot = 2 * (5 * R + 4) + 1 + 4 + 4          # two particle buffers, move tag, sort key, cell_start share
     shared = capmax * (6 * R + 4)                    # product staging / stash, product ranks
     nodes = G * (30 * R + 40 * 8 + 9 * 4 * 12)      # node fields, FP64 sums, route and counting tables
+    nodes += G * 9 * 16 * len(caps) if case_gas(deck) else 0   # product counts of the oxygen step
     solve = 2 * (ngx * ngx + ngy * ngy + 3 * G) * 8  # separable-solver matrices and work arrays
     return sum(caps) * per_slot + shared + nodes + solve + (16 << 20)
 
