@@ -92,7 +92,7 @@ struct CaseBase {
     virtual int get_timing(double *, int, long long *) = 0;
     int rf_cycles = 0, dt_pic = 0;
     int batch_refs = 0;    // batches this case belongs to (it may not be destroyed meanwhile)
-    int solver_kind = 0;   // 0 Jacobi PCG, 1 separable fast solve
+    int solver_kind = 0;   // 0 Jacobi PCG, 1 separable fast solve, 2 the same for permittivities e(x) f(y)
     int gas = 0;           // 0 Ar, 1 O2, 2 Ar/O2 (selects the collision step)
 };
 
@@ -447,11 +447,12 @@ struct Case : CaseBase {
                     HIPCHK(dalloc(&spec_part, 2 * (size_t)std::max((N + 255) / 256, field_partials(G))));
                     // an exact separable model converges in one FP64 cycle; otherwise
                     // the model error (~1e-7 relative) needs a few refinement cycles
-                    spec_cycles = sp.exact ? 1 : 4;
+                    spec_cycles = sp.cycles;
                     // a batch takes cases of one kind: exact without a shift, or not
                     spec_kind = sp.exact && !sp.shifted ? 1 : 4;
                     spectral = true;
-                    solver_kind = 1;
+                    // batches and the batching server take kind 1
+                    solver_kind = sp.product ? 2 : 1;
                 }
             }
             // the PCG's work space and launch shape (PIC_PCG_BLOCKS fixes the
@@ -1813,7 +1814,8 @@ struct Batch : BatchBase {
             Case<R> *c = cs[i];
             if (c->device != device) return fail(-70, "batch: case %zu is on another device", i);
             if (c->gas != 0) return fail(-70, "batch: case %zu is not an argon case (its step is not the fused one)", i);
-            if (!c->spectral) return fail(-70, "batch: case %zu does not use the separable field solve", i);
+            if (c->solver_kind != 1)
+                return fail(-70, "batch: case %zu does not use the separable field solve of a uniform operator", i);
             if (c->timing) return fail(-70, "batch: case %zu has stage timers on", i);
             if (c->fluid_on) return fail(-70, "batch: case %zu runs the metastable fluid", i);
             if (c->spec_kind != cs[0]->spec_kind)

@@ -109,11 +109,14 @@ int build_setup(const Deck &d, Setup<R> &s, std::string &err, bool load = true);
 // coefficients, A = cx Tx (x) I + I (x) cy Ty with Tx, Ty the 1-D second
 // difference operators (Neumann mirror or Dirichlet ends), so
 // A^-1 = (Vx (x) Vy) diag(1/(cx lx_a + cy ly_b)) (Vx^-1 (x) Vy^-1).
-// Row-major nx x nx / ny x ny FP64 matrices.
+// With permittivities e(x) f(y) the tables are those of the weighted
+// eigenproblems of both sides.  Row-major nx x nx / ny x ny FP64 matrices.
 struct Spectral {
     bool ok = false;
     bool exact = false;   // every operator entry equals the separable model bit for bit
     bool shifted = false; // ... with a non-zero shift
+    bool product = false; // non-uniform permittivity of product form
+    int cycles = 4;       // refinement cycles that reach the tolerance
     int nx = 0, ny = 0;
     double cx = 0, cy = 0, shift = 0;
     std::vector<double> Vx, Vxi, Vy, Vyi, lx, ly;

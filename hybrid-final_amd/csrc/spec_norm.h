@@ -46,7 +46,9 @@ __device__ inline bool spec_converged(double rr, double bb, double tol) {
 }
 __device__ inline void spec_decide(double rr, double bb, double tol, int last, SpecState *s, PcgResult *res) {
     const double rel = bb > 0.0 ? sqrt(rr / bb) : sqrt(rr);
-    const bool conv = spec_converged(rr, bb, tol);
+    // a zero right-hand side after a non-zero one leaves the last solution's
+    // rounding, which no relative test can pass
+    const bool conv = spec_converged(rr, bb, tol) || (last && bb == 0.0 && rr < 1e300);
     s->rel = rel;
     if (conv || last) {
         s->done = 1;

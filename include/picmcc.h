@@ -176,7 +176,8 @@ int pic_last_field_solve(pic_ctx *ctx, int *iters, int *outer, double *rel_res);
  * [7] deposit, [8] accumulators; summed over *steps steps since enabling */
 int pic_stage_timing(pic_ctx *ctx, int enable);
 int pic_stage_times(pic_ctx *ctx, double *ms, int n, long long *steps);
-/* 0 = Jacobi PCG, 1 = separable fast solve (FP64 fast-Poisson inverse in FP64 refinement) */
+/* 0 = Jacobi PCG, 1 = separable fast solve (FP64 fast-Poisson inverse in FP64 refinement),
+ * 2 = the same for permittivities that are a product e(x) f(y) (not taken into batches) */
 int pic_field_solver_kind(pic_ctx *ctx);
 /* launch shape of the persistent PCG (blocks in the grid, threads per block),
  * chosen at pic_create by timing trial solves of the case's operator (kept
