@@ -32,10 +32,23 @@
 namespace pic {
 namespace {
 
-constexpr int GT = 16;    // GEMM output tile edge
-constexpr int RB = 256;   // residual block
+constexpr int BT = 256;   // threads of a GEMM or residual block
+constexpr int RB = BT;    // unknowns of a residual block
+// blocks of a refinement cycle's launches, which loop over the work: as many
+// as the card holds at once
+constexpr int LATER_BLOCKS = 1024;
+// GEMM output tiles are 32 x 32, which halves the operand loads per product,
+// where that leaves two blocks for each of the 256 CUs and the sums are at
+// least 160 long on average over the tiles; else 16 x 16, as short sums are
+// bound by the blocks' latency and not by their loads.  A solve with small
+// tiles against large ones, in us: 24 problems of 40..120 a side (203 large
+// tiles) 106 and 105, 40 of 48..150 (427) 102 and 113, 64 of 48..224 (1060, sums
+// of 118) 153 and 158, 60 of 130 (1342) 155 and 162, 60 of 185 (2160) 278 and
+// 245, 20 of 335 (2420) 458 and 355, 2 of 620 (761) 316 and 241, 1 of 900
+// (841) 437 and 361.
+constexpr int LARGE_TILES = 512, LARGE_SUM = 160;
 
-struct GemmTask {          // one 16x16 output tile of one problem's GEMM
+struct GemmTask {          // one output tile of one problem's GEMM
     int prob, r0, c0, pad;
 };
 struct ProbDev {           // device view of one problem
@@ -64,89 +77,129 @@ __device__ inline double apply_A(const ProbDev &q, const double *x, int a, int b
     return ax;
 }
 
-// r = b - A x per block of one problem; per-block partial sums of r.r, b.b
-__global__ __launch_bounds__(RB) void k_pb_residual(const ProbDev *P, const int2 *blocks, const double *b,
-                                                    const double *x, double *r, double *part, const int *done) {
-    const int2 bl = blocks[blockIdx.x];   // (problem, first unknown of the block within the problem)
-    const ProbDev q = P[bl.x];
-    __shared__ double sh[2 * RB];
-    double rr = 0.0, bb = 0.0;
-    if (!done[bl.x]) {
+// sum of v over the block's 4 waves (every thread of wave 0 gets it), fixed order
+__device__ inline double block_sum(double v, double *sh) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+    __syncthreads();
+    return v;
+}
+
+// r = b - A x per block of one problem; per-block partial sums of r.r, b.b.
+// FIRST: the solve's start, x = 0 with r = b, read in place by the first
+// product, so only the sums and the zeros are written.  Bound by launch and
+// memory latency (7 MB: 8 us with an LDS tree over the block, 6 with shuffles).
+template <bool FIRST>
+__global__ __launch_bounds__(RB) void k_pb_residual(const ProbDev *P, const int2 *blocks, int nblk, const double *b,
+                                                    double *x, double *r, double *part, const int *done, int *left,
+                                                    int nprob) {
+    if (FIRST) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *left = nprob;
+    } else if (*left == 0) {
+        return;
+    }
+    __shared__ double sh[BT / 64];
+    for (int k = blockIdx.x; k < nblk; k += gridDim.x) {   // one pass if FIRST
+        const int2 bl = blocks[k];   // (problem, first unknown of the block within the problem)
+        if (!FIRST && done[bl.x]) continue;
+        const ProbDev q = P[bl.x];
+        double rr = 0.0, bb = 0.0;
         const int i = bl.y + (int)threadIdx.x;
         if (i < q.nx * q.ny) {
-            const int a = i / q.ny, c = i % q.ny;
             const double bi = b[q.off + i];
-            const double ri = bi - apply_A(q, x, a, c);
-            r[q.off + i] = ri;
+            double ri = bi;
+            if (FIRST) {
+                x[q.off + i] = 0.0;
+            } else {
+                ri = bi - apply_A(q, x, i / q.ny, i % q.ny);
+                r[q.off + i] = ri;
+            }
             rr = ri * ri;
             bb = bi * bi;
         }
+        rr = block_sum(rr, sh);
+        bb = block_sum(bb, sh);
+        if (threadIdx.x == 0) { part[2 * k] = rr; part[2 * k + 1] = bb; }
     }
-    sh[threadIdx.x] = rr;
-    sh[RB + threadIdx.x] = bb;
-    __syncthreads();
-    for (int o = RB / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            sh[threadIdx.x] += sh[threadIdx.x + o];
-            sh[RB + threadIdx.x] += sh[RB + threadIdx.x + o];
+}
+
+// done[] of a problem: 0 in work, 1 converged, 2 out of cycles
+// Per problem, one wave: fixed-order sum of its blocks' partials and the
+// convergence decision.  A thread a problem took 21 us for 196 partials, a
+// serial chain of loads; a wave takes 3.
+__global__ __launch_bounds__(64) void k_pb_finalize(const int *bstart, const double *part, double tol, int first,
+                                                    int last, int *done, int *left, double *rel) {
+    const int p = blockIdx.x;
+    if (!first && (*left == 0 || done[p])) return;
+    double rr = 0.0, bb = 0.0;
+    for (int k = bstart[p] + (int)threadIdx.x; k < bstart[p + 1]; k += 64) {
+        rr += part[2 * k];
+        bb += part[2 * k + 1];
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        rr += __shfl_xor(rr, o);
+        bb += __shfl_xor(bb, o);
+    }
+    if (threadIdx.x != 0) return;
+    const bool conv = bb > 0.0 ? rr <= tol * tol * bb : rr <= 1e-300;
+    rel[p] = bb > 0.0 ? sqrt(rr / bb) : sqrt(rr);
+    const int d = conv ? 1 : last ? 2 : 0;
+    done[p] = d;
+    if (d) atomicSub(left, 1);
+}
+
+// batched C = A B per problem, one tile of 16 S a side per block on the FP64
+// matrix cores (dgemm_tile_mfma, K split over the block's 4 waves); MODE
+// selects the operands:
+// 0: T1 = Vx^-1 R, 1: T2 = (T1 Vy^-T) .* dinv, 2: T1 = Vx T2, 3: x += T1 Vy^T.
+// Bound by the operand loads from L2, or by a block's chain of loads where the
+// sums are short.  The first cycle's launch has a block per tile; the later
+// ones, which usually find nothing left, loop over the tiles from fewer blocks.
+template <int MODE, int S>
+__global__ __launch_bounds__(BT) void k_pb_gemm(const ProbDev *P, const GemmTask *tasks, int ntask, const double *R,
+                                                double *T1, double *T2, double *x, const int *done, const int *left) {
+    if (*left == 0) return;
+    __shared__ double part[4][S * S * 256];
+    for (int k = blockIdx.x; k < ntask; k += gridDim.x) {
+        const GemmTask tk = tasks[k];
+        if (done[tk.prob]) continue;   // uniform over the block
+        const ProbDev q = P[tk.prob];
+        const int M = q.nx, N = q.ny;
+        const int K = (MODE == 0 || MODE == 2) ? q.nx : q.ny;
+        const double *A = MODE == 0 ? q.Vxi : MODE == 1 ? T1 + q.off : MODE == 2 ? q.Vx : T1 + q.off;
+        const double *B = MODE == 0 ? R + q.off : MODE == 1 ? q.VyiT : MODE == 2 ? T2 + q.off : q.VyT;
+        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+        if constexpr (S == 1) {
+            const v4d acc = dgemm_tile_mfma(M, N, K, A, B, tk.r0, tk.c0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) part[wv][lane * 4 + j] = acc[j];
+        } else {
+            v4d acc[4];
+            dgemm_tile_mfma2(M, N, K, A, B, tk.r0, tk.c0, acc);
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) part[wv][h * 256 + lane * 4 + j] = acc[h][j];
         }
         __syncthreads();
-    }
-    if (threadIdx.x == 0) { part[2 * blockIdx.x] = sh[0]; part[2 * blockIdx.x + 1] = sh[RB]; }
-}
-
-// per problem: fixed-order sum of its blocks' partials, convergence decision
-__global__ void k_pb_finalize(int nprob, const int *bstart, const double *part, double tol, int last, int *done,
-                              double *rel, int *status) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= nprob || done[p]) return;
-    double rr = 0.0, bb = 0.0;
-    for (int k = bstart[p]; k < bstart[p + 1]; ++k) { rr += part[2 * k]; bb += part[2 * k + 1]; }
-    const double rl = bb > 0.0 ? sqrt(rr / bb) : sqrt(rr);
-    const bool conv = bb > 0.0 ? rr <= tol * tol * bb : rr <= 1e-300;
-    rel[p] = rl;
-    if (conv || last) { done[p] = 1; status[p] = conv ? 0 : 1; }
-}
-
-// batched C = A B per problem, one 16x16 tile per block on the FP64 matrix
-// cores (dgemm_tile_mfma, K split over the block's 4 waves); MODE selects
-// the operands:
-// 0: T1 = Vx^-1 R, 1: T2 = (T1 Vy^-T) .* dinv, 2: T1 = Vx T2, 3: x += T1 Vy^T
-template <int MODE>
-__global__ __launch_bounds__(GT *GT) void k_pb_gemm(const ProbDev *P, const GemmTask *tasks, const double *R,
-                                                    double *T1, double *T2, double *x, const int *done) {
-    const GemmTask tk = tasks[blockIdx.x];
-    if (done[tk.prob]) return;   // uniform over the block
-    const ProbDev q = P[tk.prob];
-    const int M = q.nx, N = q.ny;
-    const int K = (MODE == 0 || MODE == 2) ? q.nx : q.ny;
-    const double *A = MODE == 0 ? q.Vxi : MODE == 1 ? T1 + q.off : MODE == 2 ? q.Vx : T1 + q.off;
-    const double *B = MODE == 0 ? R + q.off : MODE == 1 ? q.VyiT : MODE == 2 ? T2 + q.off : q.VyT;
-    __shared__ double part[4][256];
-    const v4d acc = dgemm_tile_mfma(M, N, K, A, B, tk.r0, tk.c0);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+        // thread t adds the four waves' accumulator slot t (lane t/4, register t%4)
+        const int t = threadIdx.x, l = t >> 2;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) part[wv][lane * 4 + j] = acc[j];
-    __syncthreads();
-    // thread t adds the four waves' accumulator slot t (lane t/4, register t%4)
-    const int t = threadIdx.x, l = t >> 2;
-    const double v = ((part[0][t] + part[1][t]) + part[2][t]) + part[3][t];
-    const int r = tk.r0 + 4 * (t & 3) + (l >> 4), c = tk.c0 + (l & 15);
-    if (r >= M || c >= N) return;
-    const size_t o = (size_t)q.off + (size_t)r * N + c;
-    if (MODE == 0) T1[o] = v;
-    else if (MODE == 1) T2[o] = v * q.dinv[(size_t)r * N + c];
-    else if (MODE == 2) T1[o] = v;
-    else x[o] += v;
-}
-
-__global__ void k_pb_begin(int nprob, int *done, int *status) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < nprob) { done[p] = 0; status[p] = 0; }
-}
-__global__ void k_pb_zero(long long n, double *x) {
-    const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (i < n) x[i] = 0.0;
+        for (int h = 0; h < S * S; ++h) {
+            const int e = h * 256 + t;
+            const double v = ((part[0][e] + part[1][e]) + part[2][e]) + part[3][e];
+            const int r = tk.r0 + 16 * (h / S) + 4 * (t & 3) + (l >> 4), c = tk.c0 + 16 * (h % S) + (l & 15);
+            if (r >= M || c >= N) continue;
+            const size_t o = (size_t)q.off + (size_t)r * N + c;
+            if (MODE == 0) T1[o] = v;
+            else if (MODE == 1) T2[o] = v * q.dinv[(size_t)r * N + c];
+            else if (MODE == 2) T1[o] = v;
+            else x[o] += v;
+        }
+        __syncthreads();   // the slots are read before the next tile's are written
+    }
 }
 
 // closed-form eigenbasis of the n x n second difference with the given ends
@@ -200,12 +253,12 @@ struct pic_pbatch {
     std::vector<long long> offs;
     ProbDev *P = nullptr;
     GemmTask *tasks = nullptr;
-    int ntask = 0;
+    int ntask = 0, tile = 16;
     int2 *blocks = nullptr;
     int nblk = 0;
     int *bstart = nullptr;
     double *b = nullptr, *x = nullptr, *r = nullptr, *T1 = nullptr, *T2 = nullptr, *part = nullptr, *rel = nullptr;
-    int *done = nullptr, *status = nullptr;
+    int *done = nullptr, *left = nullptr;   // left: problems still in work
     std::vector<void *> owned;
     std::string err;
 };
@@ -262,6 +315,7 @@ struct PbPlan {
     std::vector<GemmTask> tasks;
     std::vector<int2> blocks;
     std::vector<int> bstart;
+    int tile = 16;
     long long N = 0;
     void bind(const std::vector<const double *> &dev) {
         for (size_t p = 0; p < probs.size(); ++p) {
@@ -303,6 +357,13 @@ static int pb_plan(int nprob, const int *nx, const int *ny, const int *bc, PbPla
         pl.mats.push_back(std::move(vi));
         cache[key] = {iv, ivi};
     };
+    long long large = 0, sums = 0;
+    for (int p = 0; p < nprob; ++p) {
+        const long long t = (long long)((nx[p] + 31) / 32) * ((ny[p] + 31) / 32);
+        large += t;
+        sums += t * (((long long)nx[p] + ny[p]) / 2);
+    }
+    pl.tile = large >= LARGE_TILES && sums >= LARGE_SUM * large ? 32 : 16;
     long long off = 0;
     pl.bstart.assign(nprob + 1, 0);
     for (int p = 0; p < nprob; ++p) {
@@ -321,8 +382,8 @@ static int pb_plan(int nprob, const int *nx, const int *ny, const int *bc, PbPla
             }
         ref[4] = (int)pl.mats.size();
         pl.mats.push_back(std::move(dinv));
-        for (int r0 = 0; r0 < q.nx; r0 += GT)
-            for (int c0 = 0; c0 < q.ny; c0 += GT) pl.tasks.push_back(GemmTask{p, r0, c0, 0});
+        for (int r0 = 0; r0 < q.nx; r0 += pl.tile)
+            for (int c0 = 0; c0 < q.ny; c0 += pl.tile) pl.tasks.push_back(GemmTask{p, r0, c0, 0});
         pl.bstart[p] = (int)pl.blocks.size();
         for (int i0 = 0; i0 < q.nx * q.ny; i0 += RB) pl.blocks.push_back(make_int2(p, i0));
         pl.probs.push_back(q);
@@ -365,25 +426,35 @@ static int pb_scratch(int device, unsigned char **out) {
 // problems not yet converged.  B supplies the problem tables and work
 // vectors; b and x are the right-hand sides and the solution.
 static void pb_enqueue(const pic_pbatch &B, const double *b, double *x, double tol, int max_cycles, hipStream_t st) {
-    const int tb = 256;
-    hipLaunchKernelGGL(k_pb_begin, dim3((B.nprob + tb - 1) / tb), dim3(tb), 0, st, B.nprob, B.done, B.status);
-    hipLaunchKernelGGL(k_pb_zero, dim3((unsigned)((B.N + tb - 1) / tb)), dim3(tb), 0, st, B.N, x);
+    const ProbDev *P = B.P;
+    const dim3 blk(BT);
+    auto product = [&](auto kern, const double *R, int grid) {
+        hipLaunchKernelGGL(kern, dim3(grid), blk, 0, st, P, (const GemmTask *)B.tasks, B.ntask, R, B.T1, B.T2, x,
+                           (const int *)B.done, (const int *)B.left);
+    };
     for (int k = 0; k <= max_cycles; ++k) {
-        hipLaunchKernelGGL(k_pb_residual, dim3(B.nblk), dim3(RB), 0, st, (const ProbDev *)B.P,
-                           (const int2 *)B.blocks, b, (const double *)x, B.r, B.part, (const int *)B.done);
-        hipLaunchKernelGGL(k_pb_finalize, dim3((B.nprob + tb - 1) / tb), dim3(tb), 0, st, B.nprob,
-                           (const int *)B.bstart, (const double *)B.part, tol, k == max_cycles ? 1 : 0, B.done,
-                           B.rel, B.status);
+        const double *R = k == 0 ? b : B.r;
+        if (k == 0)
+            hipLaunchKernelGGL(k_pb_residual<true>, dim3(B.nblk), blk, 0, st, P, (const int2 *)B.blocks, B.nblk, b, x,
+                               B.r, B.part, (const int *)B.done, B.left, B.nprob);
+        else
+            hipLaunchKernelGGL(k_pb_residual<false>, dim3(std::min(B.nblk, 2 * LATER_BLOCKS)), blk, 0, st, P,
+                               (const int2 *)B.blocks, B.nblk, b, x, B.r, B.part, (const int *)B.done, B.left, B.nprob);
+        hipLaunchKernelGGL(k_pb_finalize, dim3(B.nprob), dim3(64), 0, st, (const int *)B.bstart,
+                           (const double *)B.part, tol, k == 0 ? 1 : 0, k == max_cycles ? 1 : 0, B.done, B.left, B.rel);
         if (k == max_cycles) break;
-        const dim3 g(B.ntask), blk(GT * GT);
-        hipLaunchKernelGGL(k_pb_gemm<0>, g, blk, 0, st, (const ProbDev *)B.P, (const GemmTask *)B.tasks,
-                           (const double *)B.r, B.T1, B.T2, x, (const int *)B.done);
-        hipLaunchKernelGGL(k_pb_gemm<1>, g, blk, 0, st, (const ProbDev *)B.P, (const GemmTask *)B.tasks,
-                           (const double *)B.r, B.T1, B.T2, x, (const int *)B.done);
-        hipLaunchKernelGGL(k_pb_gemm<2>, g, blk, 0, st, (const ProbDev *)B.P, (const GemmTask *)B.tasks,
-                           (const double *)B.r, B.T1, B.T2, x, (const int *)B.done);
-        hipLaunchKernelGGL(k_pb_gemm<3>, g, blk, 0, st, (const ProbDev *)B.P, (const GemmTask *)B.tasks,
-                           (const double *)B.r, B.T1, B.T2, x, (const int *)B.done);
+        const int grid = k == 0 ? B.ntask : std::min(B.ntask, LATER_BLOCKS);
+        if (B.tile == 32) {
+            product(k_pb_gemm<0, 2>, R, grid);
+            product(k_pb_gemm<1, 2>, R, grid);
+            product(k_pb_gemm<2, 2>, R, grid);
+            product(k_pb_gemm<3, 2>, R, grid);
+        } else {
+            product(k_pb_gemm<0, 1>, R, grid);
+            product(k_pb_gemm<1, 1>, R, grid);
+            product(k_pb_gemm<2, 1>, R, grid);
+            product(k_pb_gemm<3, 1>, R, grid);
+        }
     }
 }
 
@@ -414,6 +485,7 @@ int pic_pbatch_create(int nprob, const int *nx, const int *ny, const int *bc, in
     B->host = pl.probs;
     B->N = pl.N;
     B->ntask = (int)pl.tasks.size();
+    B->tile = pl.tile;
     B->nblk = (int)pl.blocks.size();
     if (pb_upload(B, &B->P, pl.probs) != hipSuccess || pb_upload(B, &B->tasks, pl.tasks) != hipSuccess ||
         pb_upload(B, &B->blocks, pl.blocks) != hipSuccess || pb_upload(B, &B->bstart, pl.bstart) != hipSuccess ||
@@ -421,7 +493,7 @@ int pic_pbatch_create(int nprob, const int *nx, const int *ny, const int *bc, in
         pb_alloc(B, &B->r, pl.N) != hipSuccess || pb_alloc(B, &B->T1, pl.N) != hipSuccess ||
         pb_alloc(B, &B->T2, pl.N) != hipSuccess || pb_alloc(B, &B->part, 2 * (size_t)B->nblk) != hipSuccess ||
         pb_alloc(B, &B->rel, nprob) != hipSuccess || pb_alloc(B, &B->done, nprob) != hipSuccess ||
-        pb_alloc(B, &B->status, nprob) != hipSuccess) {
+        pb_alloc(B, &B->left, 1) != hipSuccess) {
         g_pb_err = "device allocation failed";
         pb_destroy(B);
         return -1;
@@ -458,10 +530,10 @@ int pic_pbatch_result(pic_pbatch *B, double *x, double *rel_res) {
     if (x) PBCHK(hipMemcpyAsync(x, B->x, (size_t)B->N * sizeof(double), hipMemcpyDeviceToHost, B->st));
     if (rel_res) PBCHK(hipMemcpyAsync(rel_res, B->rel, (size_t)B->nprob * sizeof(double), hipMemcpyDeviceToHost, B->st));
     std::vector<int> stt(B->nprob);
-    PBCHK(hipMemcpyAsync(stt.data(), B->status, (size_t)B->nprob * sizeof(int), hipMemcpyDeviceToHost, B->st));
+    PBCHK(hipMemcpyAsync(stt.data(), B->done, (size_t)B->nprob * sizeof(int), hipMemcpyDeviceToHost, B->st));
     PBCHK(hipStreamSynchronize(B->st));
     int bad = 0;
-    for (int v : stt) bad += v != 0;
+    for (int v : stt) bad += v != 1;
     return bad;
 }
 
@@ -500,7 +572,7 @@ int pic_pbatch_solve_noalloc(int nprob, const int *nx, const int *ny, const int 
     const size_t oPart = region(2 * pl.blocks.size() * sizeof(double));
     const size_t oRel = region((size_t)nprob * sizeof(double));
     const size_t oDone = region((size_t)nprob * sizeof(int));
-    const size_t oStat = region((size_t)nprob * sizeof(int));
+    const size_t oLeft = region(sizeof(int));
     if (at > PB_SCRATCH_BYTES) {
         g_pb_err = "batch needs " + std::to_string(at) + " bytes of work space, more than the " +
                    std::to_string(PB_SCRATCH_BYTES) + " of the no-allocation solve";
@@ -528,6 +600,7 @@ int pic_pbatch_solve_noalloc(int nprob, const int *nx, const int *ny, const int 
     B.P = (ProbDev *)(base + oP);
     B.tasks = (GemmTask *)(base + oT);
     B.ntask = (int)pl.tasks.size();
+    B.tile = pl.tile;
     B.blocks = (int2 *)(base + oB);
     B.nblk = (int)pl.blocks.size();
     B.bstart = (int *)(base + oS);
@@ -537,15 +610,15 @@ int pic_pbatch_solve_noalloc(int nprob, const int *nx, const int *ny, const int 
     B.part = (double *)(base + oPart);
     B.rel = (double *)(base + oRel);
     B.done = (int *)(base + oDone);
-    B.status = (int *)(base + oStat);
+    B.left = (int *)(base + oLeft);
     pb_enqueue(B, b_dev, x_dev, tol, max_cycles, st);
     PBCHK(hipGetLastError());
     std::vector<int> stt(nprob);
     if (rel_res) PBCHK(hipMemcpyAsync(rel_res, B.rel, (size_t)nprob * sizeof(double), hipMemcpyDeviceToHost, st));
-    PBCHK(hipMemcpyAsync(stt.data(), B.status, (size_t)nprob * sizeof(int), hipMemcpyDeviceToHost, st));
+    PBCHK(hipMemcpyAsync(stt.data(), B.done, (size_t)nprob * sizeof(int), hipMemcpyDeviceToHost, st));
     PBCHK(hipStreamSynchronize(st));
     int bad = 0;
-    for (int v : stt) bad += v != 0;
+    for (int v : stt) bad += v != 1;
     return bad;
 }
 
