@@ -190,7 +190,7 @@ def run_pbatch(n, reps=3):
 
 
 def run_o2(steps, warmup=2):
-    """O2 chemistry (gas type 1), staged steps: 256x256 cells, dx=0.2 mm,
+    """O2 chemistry (gas type 1), whole steps: 256x256 cells, dx=0.2 mm,
     100 V, 50 mTorr, 50 particles/cell for e and O2+ and 10 for O+ and O-,
     ions colliding too; FP32 particles with the FP64-refined field solve.
     Particles are resident in HBM before the timed steps."""
@@ -209,11 +209,11 @@ def run_o2(steps, warmup=2):
     return {"workload": "O2 CCP 256x256 cells dx=0.2mm, 100 V, 50 mTorr, 50/50/10/10 particles per cell "
                         "(e, O2+, O+, O-), ions colliding, dt=T_RF/800",
             "particles": n, "steps": steps, "ms_per_step": dt * 1e3, "particle_steps_per_s": n / dt,
-            "path": "staged stages (the fused two-pass step is built for argon)"}
+            "path": "two-pass oxygen step, graph replays"}
 
 
 def run_aro2(steps, warmup=2):
-    """Ar/O2 chemistry (gas type 2), staged steps on the 512x256 workload:
+    """Ar/O2 chemistry (gas type 2), whole steps on the 512x256 workload:
     O2 20 %, 30 mTorr, 150 V, dx=0.2 mm, 100 particles/cell for e, Ar+ and
     O2+ and 20 for O+ and O- (44.6 M particles), dt=T_RF/800; FP32 particles
     with the FP64-refined field solve.  Particles are resident in HBM before
@@ -235,7 +235,7 @@ def run_aro2(steps, warmup=2):
     return {"workload": "Ar/O2 CCP 512x256 cells dx=0.2mm, O2 20 %, 30 mTorr, 150 V, 100/100/100/20/20 particles "
                         "per cell (e, Ar+, O2+, O+, O-), dt=T_RF/800",
             "particles": n1, "steps": steps, "ms_per_step": dt * 1e3, "particle_steps_per_s": n / dt,
-            "path": "staged stages with the oxygen collision step (the fused two-pass step is built for argon)"}
+            "path": "two-pass oxygen step, graph replays"}
 
 
 def run_ensemble(n, rate_hz):
@@ -384,9 +384,9 @@ def main():
     ap.add_argument("--pbatch", type=int, default=256, metavar="N",
                     help="independent Poisson problems (64^2-512^2) in the batched-solve leg (0 = skip)")
     ap.add_argument("--o2-steps", type=int, default=20, metavar="K",
-                    help="staged O2-chemistry steps timed on a 256x256 O2 case (0 = skip)")
+                    help="O2-chemistry steps timed on a 256x256 O2 case (0 = skip)")
     ap.add_argument("--aro2-steps", type=int, default=10, metavar="K",
-                    help="staged Ar/O2 steps timed on the 512x256 Ar/O2 workload (0 = skip)")
+                    help="Ar/O2 steps timed on the 512x256 Ar/O2 workload (0 = skip)")
     ap.add_argument("--ensemble", type=int, default=16, metavar="N",
                     help="cases in the served argon ensemble (Poisson arrivals; concurrent server, first-come "
                          "first-served server and one by one; 0 = skip)")

@@ -101,8 +101,8 @@ def oxygen_deck(gas=2, o2_ratio=0.2, ion_densities=None, neutral_densities=None,
     rest is Ar).  Charged-species densities default to a quasi-neutral mix
     (e 1e15, O- 2e14; positive ions make up the rest) with ppc macro-particles
     per cell for e and the molecular/atomic majority ions and ppc/5 for O+
-    and O-.  Every reaction switch is on.  Both gas types run on the GPU as
-    staged steps."""
+    and O-.  Every reaction switch is on.  Both gas types run whole steps
+    in two passes over the particles."""
     d = ccp_deck(**kw)
     ppc = kw.get("ppc", 50)
     dx = kw.get("dx", 5e-4)

@@ -135,8 +135,8 @@ int pic_dump_load(pic_ctx *ctx, const char *path);
  * for all of them over a grid that concatenates the cases' grids, from job
  * records prepared at creation; one step of the batch is one graph launch.
  * The cases must share device and precision, be argon cases on the
- * separable field solve (pic_field_solver_kind 1) with equal solve cycles,
- * and have stage timers off (-70 otherwise).  Each case gives the same bits
+ * separable field solve of a uniform operator (pic_field_solver_kind 1), all
+ * with a diagonal that rounding left exact or all with one it did not, and have stage timers off (-70 otherwise).  Each case gives the same bits
  * as when stepped alone.  A batch step is ordered after the work already
  * enqueued on the cases' streams and before work enqueued on them later, so
  * pic_sync / pic_get_* on a case see the batch's steps.  A case stepped
@@ -179,10 +179,11 @@ int pic_stage_times(pic_ctx *ctx, double *ms, int n, long long *steps);
 /* 0 = Jacobi PCG, 1 = separable fast solve (FP64 fast-Poisson inverse in FP64 refinement),
  * 2 = the same for permittivities that are a product e(x) f(y) (not taken into batches) */
 int pic_field_solver_kind(pic_ctx *ctx);
-/* launch shape of the persistent PCG (blocks in the grid, threads per block),
+/* launch shape of the persistent PCG (blocks in the grid, threads per block):
+ * by the number of unknowns where the vectors fit the registers, otherwise
  * chosen at pic_create by timing trial solves of the case's operator (kept
- * per operator size for the process; the environment variable
- * PIC_PCG_BLOCKS fixes the grid instead); 0, 0 with the separable solve.
+ * per operator size for the process); the environment variable
+ * PIC_PCG_BLOCKS fixes the grid instead; 0, 0 with the separable solve.
  * No counterpart in the reference, whose PCG_float launch is fixed. */
 int pic_field_solver_shape(pic_ctx *ctx, int *blocks, int *threads);
 
@@ -232,7 +233,8 @@ void pic_setup_close(pic_setup_h *h);
  * the deck's object under "Collision_On_Off", then every reaction key in
  * reaction order, newline-separated (src/start.c:1003-1420); NULL for an
  * unknown type.  For gas types 1 and 2 pic_mcc applies the O2 or Ar/O2
- * collision step, and pic_step runs the stages one by one. */
+ * collision step, and pic_step runs it inside whole steps of two passes over
+ * the particles. */
 const char *pic_reaction_names(int gas);
 
 /* ---------------- reference-named zero-argument shims ---------------- */
